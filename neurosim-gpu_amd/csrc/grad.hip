@@ -15,14 +15,14 @@
 // output, as in torch.
 //
 // Launches: j = W @ s again (the row-block product, as in ns_csr_spmm), the
-// elementwise backward (one lane per neuron, columns in order, so the
-// parameter sums are deterministic), the transposed product added into the
-// state gradient (one wavefront per source neuron over its out-edges) and the
-// weight gradient (one wavefront per destination row; each edge sums its
-// columns in order).  No atomics: every result has a single writer.
+// elementwise backward (one lane per neuron and column), the transposed product
+// added into the state gradient (a group of lanes per source neuron over its
+// out-edges) and the weight gradient (a group of lanes per destination row).
+// No atomics: every result has a single writer.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "ns_common.h"
 #include "ns_host.h"
@@ -31,7 +31,6 @@ namespace ns {
 namespace {
 
 constexpr int kGradThreads = 256;
-constexpr int kGradChunk = 8;   // columns per pass of the wavefront kernels
 constexpr int kGradUnroll = 4;  // edges per lane per round of the edge loops
 
 struct GradArgs {
@@ -45,16 +44,26 @@ struct GradArgs {
   float* gp[6];
 };
 
+// One lane per (neuron, column), LB lanes per neuron; lane q takes columns q,
+// q + LB, ...  The parameter gradients sum a neuron's columns: each lane its
+// own in order, then an xor butterfly over the LB lanes, so they are
+// repeatable.  Bound by latency (three reads deep) at mid sizes; one lane per
+// neuron walking its columns left three quarters of the lanes' loads in a
+// serial chain (N=50k, B=8: 13.6 us; 196 workgroups).
+template <int LB>
 __global__ __launch_bounds__(kGradThreads) void advance_backward_kernel(GradArgs A) {
 #pragma clang fp contract(off)
-  const int64_t n = static_cast<int64_t>(blockIdx.x) * kGradThreads + threadIdx.x;
-  if (n >= A.N) return;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kGradThreads + threadIdx.x;
+  const int64_t n = t / LB;
+  const int q = static_cast<int>(t % LB);
+  if (n >= A.N) return;  // the LB lanes of a neuron leave together
   const NeuronParams P = load_params(A.p, n);
   float g_alpha = 0.0f, g_gain = 0.0f, g_rho_d = 0.0f, g_rho_a = 0.0f, g_c = 0.0f, g_k = 0.0f;
-  for (int64_t b = 0; b < A.B; ++b) {
+  for (int64_t b = q; b < A.B; b += LB) {
     const float j = A.j[n * A.B + b];
     const float s = A.s.get(b, n), d = A.d.get(b, n), a = A.a.get(b, n);
     const float u = A.u.get(b, n), v = A.v.get(b, n);
+    const float gS = A.gs_up.get(b, n), gD = A.gd_up.get(b, n), gA = A.ga_up.get(b, n);
     // Forward, rounded as the tick rounds it.
     const float t1 = tanhf(j + v);
     const float dn = P.rho_d * d + (1.0f - P.rho_d) * t1;
@@ -65,7 +74,6 @@ __global__ __launch_bounds__(kGradThreads) void advance_backward_kernel(GradArgs
     const float pre = P.alpha * s + (1.0f - P.alpha) * eq;
     const float sn = clamp01(pre);
     // Backward.
-    const float gS = A.gs_up.get(b, n), gD = A.gd_up.get(b, n), gA = A.ga_up.get(b, n);
     g_rho_a += gA * (a - sn);
     const float g_sn = gS + (1.0f - P.rho_a) * gA;
     const float g_pre = (pre >= 0.0f && pre <= 1.0f) ? g_sn : 0.0f;
@@ -85,89 +93,189 @@ __global__ __launch_bounds__(kGradThreads) void advance_backward_kernel(GradArgs
     if (A.gv.data) A.gv.put(b, n, g_x1);
     A.gj[n * A.B + b] = (1.0f - P.coupling) * g_x2 + g_x1;
   }
-  const float sums[6] = {g_alpha, g_gain, g_rho_d, g_rho_a, g_c, g_k};
+  float sums[6] = {g_alpha, g_gain, g_rho_d, g_rho_a, g_c, g_k};
+#pragma unroll
+  for (int off = LB / 2; off > 0; off >>= 1) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) sums[i] += __shfl_xor(sums[i], off, 64);
+  }
 #pragma unroll
   for (int i = 0; i < 6; ++i)
-    if (A.gp[i]) A.gp[i][n] = sums[i];
+    if (q == 0 && A.gp[i]) A.gp[i][n] = sums[i];
 }
 
-__device__ __forceinline__ float wave_sum(float x) {
+// The two edge kernels below give each row (a source, or a destination) a
+// power-of-two group of lanes: LPE lanes per edge, VL neighbouring columns each
+// (one 4 * VL byte load of a neuron-major row; VL = 1 takes any strides), and
+// `edge_lanes` edges at a time, kGradUnroll rounds of them in flight.  The host
+// picks edge_lanes so that a row of average length is about one round
+// (edge_lanes_for).  A wavefront per row, every lane walking its edge's columns
+// by itself, left two thirds of the lanes idle at 20 edges per row and read
+// each gathered row in 4-byte pieces.
+
+template <int VL>
+__device__ __forceinline__ void load_row(const float* at, float x[VL]) {
+  typedef float vec __attribute__((ext_vector_type(VL == 1 ? 2 : VL)));
+  if constexpr (VL == 1) {
+    x[0] = *at;
+  } else {
+    const vec y = *reinterpret_cast<const vec*>(at);
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
+    for (int k = 0; k < VL; ++k) x[k] = y[k];
+  }
 }
 
 // gs[b, c] += sum over out-edges e of source c of w[owi[e]] * gj[dst[e], b].
+template <int VL, int LPE>
 __global__ __launch_bounds__(kGradThreads) void transposed_product_kernel(
     const int32_t* out_rowptr, const int32_t* dst, const int32_t* owi, const float* w,
-    const float* w_out, const float* gj, int64_t N, int64_t B, OutPlane gs) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * (kGradThreads / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (c >= N) return;
+    const float* w_out, const float* gj, int64_t N, int64_t B, OutPlane gs, int edge_lanes_log2) {
+  constexpr int kCols = VL * LPE;
+  const int edge_lanes = 1 << edge_lanes_log2;
+  const int group = LPE << edge_lanes_log2;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kGradThreads + threadIdx.x;
+  const int64_t c = t >> (__builtin_ctz(LPE) + edge_lanes_log2);
+  if (c >= N) return;  // the lanes of a group leave together
+  const int lane = static_cast<int>(t & (group - 1));
+  const int q = lane & (LPE - 1), el = lane / LPE;
   const int32_t e0 = out_rowptr[c], e1 = out_rowptr[c + 1];
-  for (int64_t b0 = 0; b0 < B; b0 += kGradChunk) {
-    float acc[kGradChunk];
+  for (int64_t b0 = 0; b0 < B; b0 += kCols) {
+    const int64_t b = b0 + q * VL;
+    const bool have = b < B;
+    float acc[VL];
 #pragma unroll
-    for (int q = 0; q < kGradChunk; ++q) acc[q] = 0.0f;
-    // kGradUnroll edges per lane per round, every load of a round issued before
-    // the first multiply (an edge past the row's end rereads the row's last edge
-    // and adds nothing), so a round waits on memory once.
-    for (int32_t e = e0 + lane; e < e1; e += 64 * kGradUnroll) {
-      float weight[kGradUnroll];
-      int64_t t[kGradUnroll];
+    for (int k = 0; k < VL; ++k) acc[k] = 0.0f;
+    // Every load of a round is issued before the first multiply (an edge past
+    // the row's end rereads the row's last edge and adds nothing), so a round
+    // waits on memory twice: indices and weights, then the gathered rows.
+    for (int32_t e = e0 + el; e < e1; e += edge_lanes * kGradUnroll) {
+      float weight[kGradUnroll], g[kGradUnroll][VL];
+      int64_t to[kGradUnroll];
 #pragma unroll
       for (int u = 0; u < kGradUnroll; ++u) {
-        const int32_t at = min(e + 64 * u, e1 - 1);
+        const int32_t at = min(e + edge_lanes * u, e1 - 1);
         // Source-major weights stream; otherwise each one is a gather into the CSR order.
         weight[u] = w_out ? w_out[at] : w[owi[at]];
-        t[u] = dst[at];
+        to[u] = dst[at];
       }
+#pragma unroll
+      for (int u = 0; u < kGradUnroll; ++u) load_row<VL>(gj + to[u] * B + (have ? b : 0), g[u]);
 #pragma unroll
       for (int u = 0; u < kGradUnroll; ++u) {
-        if (e + 64 * u >= e1) break;
+        if (e + edge_lanes * u >= e1) break;
 #pragma unroll
-        for (int q = 0; q < kGradChunk; ++q)
-          if (b0 + q < B) acc[q] = __builtin_fmaf(weight[u], gj[t[u] * B + b0 + q], acc[q]);
+        for (int k = 0; k < VL; ++k) acc[k] = __builtin_fmaf(weight[u], g[u][k], acc[k]);
       }
     }
+    for (int off = LPE; off < group; off <<= 1) {
 #pragma unroll
-    for (int q = 0; q < kGradChunk; ++q) {
-      const float total = wave_sum(acc[q]);
-      if (lane == 0 && b0 + q < B) {
-        float* at = gs.data + (b0 + q) * gs.sb + c * gs.sn;
-        *at = *at + total;
+      for (int k = 0; k < VL; ++k) acc[k] += __shfl_xor(acc[k], off, 64);
+    }
+    if (el == 0 && have) {
+#pragma unroll
+      for (int k = 0; k < VL; ++k) {
+        float* at = gs.data + (b + k) * gs.sb + c * gs.sn;
+        *at = *at + acc[k];
       }
     }
   }
 }
 
-// gw[e] = sum over columns b (in order) of gj[row, b] * s[b, col[e]], for the
-// edges e of each destination row.
+// gw[e] = sum over columns b of gj[row, b] * s[b, col[e]], for the edges e of
+// each destination row: each lane sums its columns in order, the LPE lanes of
+// an edge by an xor butterfly.
+template <int VL, int LPE>
 __global__ __launch_bounds__(kGradThreads) void weight_gradient_kernel(
     const int32_t* rowptr, const int32_t* col, const float* gj, Plane s, int64_t N, int64_t B,
-    float* gw) {
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * (kGradThreads / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (r >= N) return;
+    float* gw, int edge_lanes_log2) {
+  constexpr int kCols = VL * LPE;
+  const int edge_lanes = 1 << edge_lanes_log2;
+  const int group = LPE << edge_lanes_log2;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kGradThreads + threadIdx.x;
+  const int64_t r = t >> (__builtin_ctz(LPE) + edge_lanes_log2);
+  if (r >= N) return;  // the lanes of a group leave together
+  const int lane = static_cast<int>(t & (group - 1));
+  const int q = lane & (LPE - 1), el = lane / LPE;
   const int32_t e0 = rowptr[r], e1 = rowptr[r + 1];
-  // kGradUnroll edges per lane per round: the round's column indices load
-  // together, then their state gathers, then the stores.
-  for (int32_t e = e0 + lane; e < e1; e += 64 * kGradUnroll) {
+  // A round's column indices load together, then their state gathers, then the
+  // stores.
+  for (int32_t e = e0 + el; e < e1; e += edge_lanes * kGradUnroll) {
     int64_t c[kGradUnroll];
 #pragma unroll
-    for (int u = 0; u < kGradUnroll; ++u) c[u] = col[min(e + 64 * u, e1 - 1)];
+    for (int u = 0; u < kGradUnroll; ++u) c[u] = col[min(e + edge_lanes * u, e1 - 1)];
     float sum[kGradUnroll];
 #pragma unroll
     for (int u = 0; u < kGradUnroll; ++u) sum[u] = 0.0f;
-    for (int64_t b = 0; b < B; ++b) {
-      const float g = gj[r * B + b];
+    for (int64_t b0 = 0; b0 < B; b0 += kCols) {
+      const int64_t b = b0 + q * VL;
+      const bool have = b < B;
+      float g[VL], x[kGradUnroll][VL];
+      load_row<VL>(gj + r * B + (have ? b : 0), g);
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u) sum[u] = __builtin_fmaf(g, s.get(b, c[u]), sum[u]);
+      for (int u = 0; u < kGradUnroll; ++u)
+        load_row<VL>(s.data + (have ? b : 0) * s.sb + c[u] * s.sn, x[u]);
+#pragma unroll
+      for (int k = 0; k < VL; ++k) g[k] = have ? g[k] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < kGradUnroll; ++u) {
+#pragma unroll
+        for (int k = 0; k < VL; ++k)
+          sum[u] = have ? __builtin_fmaf(g[k], x[u][k], sum[u]) : sum[u];
+      }
+    }
+#pragma unroll
+    for (int off = 1; off < LPE; off <<= 1) {
+#pragma unroll
+      for (int u = 0; u < kGradUnroll; ++u) sum[u] += __shfl_xor(sum[u], off, 64);
     }
 #pragma unroll
     for (int u = 0; u < kGradUnroll; ++u)
-      if (e + 64 * u < e1) gw[e + 64 * u] = sum[u];
+      if (q == 0 && e + edge_lanes * u < e1) gw[e + edge_lanes * u] = sum[u];
   }
+}
+
+// log2 of the edges a row's group takes at a time: the smallest power of two for
+// which kGradUnroll of them cover a row of average length, at most what fits
+// one wavefront beside the LPE lanes of an edge.
+inline int edge_lanes_for(int64_t edges, int64_t rows, int lpe) {
+  int lg = 0;
+  while ((lpe << lg) < 64 && (int64_t{kGradUnroll} << lg) * rows < edges) ++lg;
+  return lg;
+}
+
+struct EdgeForm {
+  int vl, lpe;
+};
+
+// The edge kernels' form for a batch: VL = 4 (2 at B = 2) where whole neuron-major
+// rows can be loaded, else one column per lane.
+inline EdgeForm edge_form(int64_t batch, bool whole_rows) {
+  if (whole_rows && batch == 2) return {2, 1};
+  if (whole_rows && batch % 4 == 0) return {4, batch == 4 ? 1 : batch == 8 ? 2 : 4};
+  return {1, batch <= 1 ? 1 : batch == 2 ? 2 : batch <= 4 ? 4 : batch <= 8 ? 8 : 16};
+}
+
+template <typename F>
+inline void with_edge_form(EdgeForm form, F&& launch) {
+  if (form.vl == 4) {
+    if (form.lpe == 1) launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+    else if (form.lpe == 2) launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+  } else if (form.vl == 2) {
+    launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
+  } else {
+    switch (form.lpe) {
+      case 1: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}); break;
+      case 2: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{}); break;
+      case 4: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{}); break;
+      case 8: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{}); break;
+      default: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
+    }
+  }
+}
+
+inline unsigned lanes_grid(int64_t rows, int group) {
+  return static_cast<unsigned>((rows * group + kGradThreads - 1) / kGradThreads);
 }
 
 }  // namespace
@@ -266,10 +374,17 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
       if (overlaps(part, outs[o]))
         return fail("the transposed panels' partials overlap a gradient plane");
   }
-  const unsigned per_neuron = static_cast<unsigned>((n + kGradThreads - 1) / kGradThreads);
-  const unsigned per_row = static_cast<unsigned>((n + kGradThreads / 64 - 1) / (kGradThreads / 64));
-  advance_backward_kernel<<<per_neuron, kGradThreads, 0, s>>>(G);
+  switch (batch <= 1 ? 1 : batch <= 2 ? 2 : batch <= 4 ? 4 : batch <= 8 ? 8 : 16) {
+    case 1: advance_backward_kernel<1><<<lanes_grid(n, 1), kGradThreads, 0, s>>>(G); break;
+    case 2: advance_backward_kernel<2><<<lanes_grid(n, 2), kGradThreads, 0, s>>>(G); break;
+    case 4: advance_backward_kernel<4><<<lanes_grid(n, 4), kGradThreads, 0, s>>>(G); break;
+    case 8: advance_backward_kernel<8><<<lanes_grid(n, 8), kGradThreads, 0, s>>>(G); break;
+    default: advance_backward_kernel<16><<<lanes_grid(n, 16), kGradThreads, 0, s>>>(G);
+  }
   if (a.matrix.n_edges > 0) {
+    // gj is neuron-major; whole rows of it load at once when it is aligned.
+    const bool gj_rows = batch % 4 == 0 ? reinterpret_cast<uintptr_t>(gj) % 16 == 0
+                                        : batch == 2 && reinterpret_cast<uintptr_t>(gj) % 8 == 0;
     if (a.transposed_panels) {
       // d_state += W^T @ gj on the transposed matrix's panel layout (checked
       // before the first launch).
@@ -277,13 +392,27 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
         return fail_launch("tick backward", e);
       if (int rc = panel_step(transposed, s, 2, true)) return rc;
     } else {
-      transposed_product_kernel<<<per_row, kGradThreads, 0, s>>>(
-          a.out_rowptr, a.dst, a.out_weight_index, static_cast<const float*>(a.matrix.weight),
-          a.out_weight, gj, n, batch, out_plane(a.d_state));
+      const EdgeForm form = edge_form(batch, gj_rows);
+      const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe);
+      with_edge_form(form, [&](auto vl, auto lpe) {
+        transposed_product_kernel<vl(), lpe()><<<lanes_grid(n, form.lpe << lg), kGradThreads, 0, s>>>(
+            a.out_rowptr, a.dst, a.out_weight_index, static_cast<const float*>(a.matrix.weight),
+            a.out_weight, gj, n, batch, out_plane(a.d_state), lg);
+      });
     }
-    if (a.d_weight)
-      weight_gradient_kernel<<<per_row, kGradThreads, 0, s>>>(
-          a.matrix.rowptr, a.matrix.col, gj, plane(a.state, a.state.data), n, batch, a.d_weight);
+    if (a.d_weight) {
+      // The state's rows load whole when it is neuron-major and aligned too.
+      const int64_t width = batch % 4 == 0 ? 4 : 2;
+      const bool s_rows = gj_rows && a.state.stride_b == 1 && a.state.stride_n % width == 0 &&
+                          reinterpret_cast<uintptr_t>(a.state.data) % (4 * width) == 0;
+      const EdgeForm form = edge_form(batch, s_rows);
+      const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe);
+      with_edge_form(form, [&](auto vl, auto lpe) {
+        weight_gradient_kernel<vl(), lpe()><<<lanes_grid(n, form.lpe << lg), kGradThreads, 0, s>>>(
+            a.matrix.rowptr, a.matrix.col, gj, plane(a.state, a.state.data), n, batch, a.d_weight,
+            lg);
+      });
+    }
   }
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return fail_launch("tick backward", err);

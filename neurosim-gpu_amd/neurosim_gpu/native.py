@@ -981,16 +981,16 @@ class NativeExtension:
                                   else _OutPlane(None, 0, 0))
         d_weight = torch.empty_like(weight) if need_weight else None
         args.d_weight = d_weight.data_ptr() if d_weight is not None and weight.numel() else None
-        # The wanted parameter gradients and the workspace share one allocation.
+        # The workspace and the wanted parameter gradients share one allocation, the
+        # workspace first: the kernels load whole rows of it when it is 16-byte aligned.
         wanted = [i for i, want in enumerate(need_params) if want]
         work = int(self.lib.ns_step_backward_workspace_floats(n, batch))
-        block = torch.empty(len(wanted) * n + work, dtype=torch.float32, device=state.device)
+        block = torch.empty(work + len(wanted) * n, dtype=torch.float32, device=state.device)
         d_params = [None] * 6
         for k, i in enumerate(wanted):
-            d_params[i] = block[k * n:(k + 1) * n]
+            d_params[i] = block[work + k * n:work + (k + 1) * n]
             args.d_params[i] = d_params[i].data_ptr()
-        workspace = block[len(wanted) * n:]
-        args.workspace = workspace.data_ptr() if workspace.numel() else None
+        args.workspace = block.data_ptr() if work else None
         stream = torch.cuda.current_stream(state.device).cuda_stream
         _raise_on(self.lib.ns_dendritic_step_backward(ctypes.byref(args), stream), self.lib)
         return (*planes[:3], d_drive, d_dendritic, d_weight, d_params)
@@ -1369,14 +1369,14 @@ class PreparedBackward:
         planes = storage.transpose(1, 2).unbind(0)
         d_weight = torch.empty_like(weight) if need_weight else None
         wanted = [i for i, want in enumerate(need_params) if want]
-        block = torch.empty(len(wanted) * n + self._work, dtype=torch.float32,
-                            device=self.device)
+        work = self._work               # first in the block, so 16-byte aligned
+        block = torch.empty(work + len(wanted) * n, dtype=torch.float32, device=self.device)
         d_params = [None] * 6
         param_ptrs = [0] * 6
         for k, i in enumerate(wanted):
-            d_params[i] = block[k * n:(k + 1) * n]
+            d_params[i] = block[work + k * n:work + (k + 1) * n]
             param_ptrs[i] = d_params[i].data_ptr()
-        workspace_ptr = block.data_ptr() + 4 * len(wanted) * n if self._work else 0
+        workspace_ptr = block.data_ptr() if work else 0
         _POINTERS11.pack_into(args, _GRAD_POINTERS,
                               d_weight.data_ptr() if d_weight is not None and weight.numel() else 0,
                               *param_ptrs, workspace_ptr, current_ptr, out_weight_ptr,
