@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define NS_ABI_VERSION 19
+#define NS_ABI_VERSION 20
 
 /* Return codes. */
 #define NS_OK 0
@@ -363,7 +363,14 @@ typedef struct ns_step_grad_args {
                                   d_state) instead of the out-edge walk; out_weight is
                                   then unused.  Its partials workspace must not overlap
                                   the gradient planes or the workspace. */
+  int32_t flags;               /* NS_GRAD_* */
+  int32_t reserved;
 } ns_step_grad_args;
+
+/* ns_step_grad_args flag: the caller does not want the gradient of the state
+ * (its recorded state needs none), so the transposed product W^T @ g is not
+ * run; `d_state` is still required and receives the update's own part only. */
+#define NS_GRAD_NO_STATE 1
 
 /* Arguments of one weight encoding (fp8 e4m3 or NVFP4 CSR payload). */
 typedef struct ns_encode_args {

@@ -310,6 +310,8 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
     return fail("the source-major view (out_rowptr, dst, out_weight_index) is required");
   if (!a.workspace) return fail("a workspace of 2*B*N floats is required");
   if (a.transposed_panels && batch > 2) return fail("transposed panels need batch 1 or 2");
+  if (a.flags & ~NS_GRAD_NO_STATE) return fail("unknown backward flags %d", a.flags);
+  const bool want_state = (a.flags & NS_GRAD_NO_STATE) == 0;
   const Extent outs[5] = {extent(a.d_state, batch, n), extent(a.d_dendrite, batch, n),
                           extent(a.d_adaptation, batch, n), extent(a.d_drive, batch, n),
                           extent(a.d_dendritic_drive, batch, n)};
@@ -356,7 +358,7 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
   for (int i = 0; i < 6; ++i) G.gp[i] = a.d_params[i];
   // The transposed product on panels: W^T @ gj added into d_state.
   ns_step_args transposed{};
-  if (a.transposed_panels && a.matrix.n_edges > 0) {
+  if (want_state && a.transposed_panels && a.matrix.n_edges > 0) {
     transposed.n_neurons = n; transposed.batch = batch;
     transposed.state = ns_plane{gj, 1, batch, 0.0f};
     transposed.matrix.n_rows = n; transposed.matrix.n_edges = a.matrix.n_edges;
@@ -385,13 +387,13 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
     // gj is neuron-major; whole rows of it load at once when it is aligned.
     const bool gj_rows = batch % 4 == 0 ? reinterpret_cast<uintptr_t>(gj) % 16 == 0
                                         : batch == 2 && reinterpret_cast<uintptr_t>(gj) % 8 == 0;
-    if (a.transposed_panels) {
+    if (want_state && a.transposed_panels) {
       // d_state += W^T @ gj on the transposed matrix's panel layout (checked
       // before the first launch).
       if (const hipError_t e = hipGetLastError(); e != hipSuccess)
         return fail_launch("tick backward", e);
       if (int rc = panel_step(transposed, s, 2, true)) return rc;
-    } else {
+    } else if (want_state) {
       const EdgeForm form = edge_form(batch, gj_rows);
       const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe);
       with_edge_form(form, [&](auto vl, auto lpe) {

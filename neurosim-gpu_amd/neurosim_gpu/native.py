@@ -37,7 +37,7 @@ import numpy as np
 import torch
 
 _LIB_NAME = "libneurosim_hip.so"
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 WEIGHT_F32, WEIGHT_F16, WEIGHT_E4M3, WEIGHT_NVFP4 = 0, 1, 2, 3
 _PLAN_CACHE = 64   # row plans kept per extension (one per live topology and batch width)
@@ -138,7 +138,10 @@ class _StepGradArgs(ctypes.Structure):
                 ("d_state", _OutPlane), ("d_dendrite", _OutPlane), ("d_adaptation", _OutPlane),
                 ("d_drive", _OutPlane), ("d_dendritic_drive", _OutPlane),
                 ("d_weight", _c_ptr), ("d_params", _c_ptr * 6), ("workspace", _c_ptr),
-                ("current", _c_ptr), ("out_weight", _c_ptr), ("transposed_panels", _c_ptr)]
+                ("current", _c_ptr), ("out_weight", _c_ptr), ("transposed_panels", _c_ptr),
+                ("flags", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+
+GRAD_NO_STATE = 1        # NS_GRAD_NO_STATE
 
 
 class _EncodeArgs(ctypes.Structure):
@@ -1284,7 +1287,9 @@ class PreparedBackward:
     and the optional source-major weights, allocates the gradient planes (one
     allocation), the weight gradient and the parameter gradients with the
     workspace (one allocation), writes the per-call words and launches.  The
-    results equal ``NativeExtension.dendritic_step_backward`` on the same inputs."""
+    results equal ``NativeExtension.dendritic_step_backward`` on the same inputs.
+    ``need_state=False`` leaves out the transposed product: the returned d_state
+    is then the update's own part, for a caller that drops it."""
 
     def __init__(self, extension: "NativeExtension", state: torch.Tensor, params, rowptr, col,
                  weight, out_rowptr, dst, weight_index):
@@ -1328,7 +1333,7 @@ class PreparedBackward:
                  dendritic_scalar, grad_state, grad_dendrite, grad_adaptation, *,
                  need_drive=False, need_dendritic=False, need_weight=False,
                  need_params=(False,) * 6, out_weight=None, current=None,
-                 transposed_panels=None):
+                 transposed_panels=None, need_state=True):
         _check_state(state)
         if state.device != self.device:
             raise RuntimeError("all tensors must be on the state's CUDA device")
@@ -1382,6 +1387,7 @@ class PreparedBackward:
                               *param_ptrs, workspace_ptr, current_ptr, out_weight_ptr,
                               ctypes.addressof(transposed_panels) if transposed_panels is not None
                               else 0)
+        args.flags = 0 if need_state else GRAD_NO_STATE
         _raise_on(self.lib.ns_dendritic_step_backward(self._ref, current_stream(self.device)),
                   self.lib)
         d_drive = planes[3] if need_drive else None

@@ -31,8 +31,8 @@ import torch
 from .compartmental import DendriticDynamics, DendriticMatrixRuntime, DendriticPELSRuntime
 from .native import (BAND_WIDTH, EVENT_ACTIVITY_SLOTS, EVENT_ACTIVITY_STRIDE, BandLayout,
                      NativeExtension, PanelLayout, PreparedAccumulate, PreparedBackward,
-                     PreparedEvent, PreparedTick, encode_weights,
-                     load_native_extension, panel_geometry)
+                     PreparedEvent, PreparedTick, _neuron_major, encode_weights,
+                     load_native_extension, new_planes, panel_geometry)
 from .topology import SparseTopology
 
 
@@ -151,13 +151,16 @@ class TransposedPanels:
     """Column-panel layout of the transposed matrix, for the backward's W^T @ g.
 
     Its rows are the sources (``out_rowptr``, ``dst``: the source-major view)
-    and its slots name CSR positions through ``out_weight_index``.  On the
-    first request for a weight version the plan is indexed (NS_PANEL_INDEXED):
-    the kernel reads each slot's weight from the CSR-order weights through
-    that position, so a weight version used once (an optimizer step before
-    every backward) needs no copy.  The slot-order copy, one random read per
-    edge, is made on the second request (backpropagation through several
-    ticks, or repeated passes on fixed weights), and streamed after that.
+    and its slots name CSR positions through ``out_weight_index``.  When a
+    weight version is used once (an optimizer step before every backward) the
+    plan is indexed (NS_PANEL_INDEXED): the kernel reads each slot's weight
+    from the CSR-order weights through that position, and no copy is made.
+    The slot-order copy, one random read per edge, is made on the first request
+    when ``expect`` has announced two or more products of the version
+    (backpropagation through several ticks), else on the second (repeated passes
+    on fixed weights), and streamed after that.  N=166k, M=25M: an indexed
+    product takes 327 us, the copy 413 and a streamed product 33, so two
+    products cost 479 us with the copy made at once and 773 with it made late.
     Built on the host from the source-major view (set-up only, like the
     forward's layout)."""
 
@@ -170,19 +173,30 @@ class TransposedPanels:
         owi = topology.out_weight_index.to(device=device, dtype=torch.int32)
         self.layout.perm = torch.where(perm >= 0, owi[perm.clamp(min=0).long()],
                                        perm).to(torch.int32).contiguous()
-        self._key, self._source, self._seen = None, None, 0
+        self._key, self._source, self._seen, self._expected = None, None, 0, 0
         self._indexed = None
 
-    def plan(self, weight: torch.Tensor):
-        """The plan struct for ``weight`` (float32, CSR order): on the first
-        request for a weight version the indexed plan, whose slots carry CSR
-        edge numbers so the kernel reads ``weight`` in place; from the second on,
-        ``weight`` gathered into slot order once."""
+    def _version(self, weight: torch.Tensor) -> tuple:
         key = _weight_key(weight)
         if key != self._key or self._source is not weight:
-            self._key, self._source, self._seen = key, weight, 0
+            self._key, self._source, self._seen, self._expected = key, weight, 0, 0
+        return key
+
+    def expect(self, weight: torch.Tensor) -> None:
+        """One more recorded tick of this weight version whose backward asks for
+        a product."""
+        self._version(weight)
+        self._expected += 1
+
+    def plan(self, weight: torch.Tensor):
+        """The plan struct for ``weight`` (float32, CSR order): the indexed plan,
+        whose slots carry CSR edge numbers so the kernel reads ``weight`` in place,
+        or ``weight`` gathered into slot order once (see above)."""
+        key = self._version(weight)
         self._seen += 1
-        if self._seen < 2:
+        # No copy inside a capture: it would be filled only when the graph replays.
+        if (self._seen < 2 and self._expected < 2) or (
+                self.layout._slot_key != key and torch.cuda.is_current_stream_capturing()):
             if self._indexed is None:
                 self._indexed = self.layout.indexed_plan_struct()
             return self._indexed
@@ -198,7 +212,10 @@ class _NativeTick(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, info, state, dendrite, adaptation, weight, drive, dendritic_drive, *params):
-        _, _, us, vs, tick, _, _, _ = info
+        _, _, us, vs, tick, _, _, _, by_neuron = info
+        if by_neuron and not _neuron_major(state):
+            # One gathered run per edge for the forward and the weight gradient.
+            state = new_planes(1, *state.shape, state)[0].copy_(state)
         # The launch arguments were prepared (and validated) for this weight, plan
         # and these parameters; j = W @ s is kept for the backward, which then
         # needs no product of its own.
@@ -215,7 +232,7 @@ class _NativeTick(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_state, grad_dendrite, grad_adaptation):
-        extension, topology, us, vs, _, source_major, transposed, cache = ctx.info
+        extension, topology, us, vs, _, source_major, transposed, cache, _ = ctx.info
         saved = list(ctx.saved_tensors)
         state, dendrite, adaptation, weight = saved[:4]
         params = saved[4:10]
@@ -223,9 +240,12 @@ class _NativeTick(torch.autograd.Function):
         drive = next(rest) if ctx.has_drive[0] else None
         dendritic_drive = next(rest) if ctx.has_drive[1] else None
         needs = ctx.needs_input_grad
-        panels = transposed.plan(weight) if transposed is not None else None
-        out_weight = (None if panels is not None
-                      else source_major.get(weight, topology.out_weight_index))
+        # A start state that needs no gradient needs no transposed product either.
+        panels = out_weight = None
+        if needs[1]:
+            panels = transposed.plan(weight) if transposed is not None else None
+            out_weight = (None if panels is not None
+                          else source_major.get(weight, topology.out_weight_index))
         fixed = (topology.in_rowptr, topology.in_col, weight, topology.out_rowptr,
                  topology.dst, topology.out_weight_index)
         prepared = cache[0]
@@ -237,7 +257,8 @@ class _NativeTick(torch.autograd.Function):
             grad_dendrite, grad_adaptation, need_drive=bool(needs[5]),
             need_dendritic=bool(needs[6]), need_weight=bool(needs[4]),
             need_params=tuple(bool(x) for x in needs[7:13]),
-            out_weight=out_weight, current=ctx.current, transposed_panels=panels)
+            out_weight=out_weight, current=ctx.current, transposed_panels=panels,
+            need_state=bool(needs[1]))
         ctx.current = None
         return (None, d_state if needs[1] else None, d_dendrite if needs[2] else None,
                 d_adaptation if needs[3] else None, d_weight, d_drive, d_dendritic, *d_params)
@@ -289,6 +310,13 @@ def bands_pay_off(n_neurons: int, batch: int) -> bool:
     """Whether "auto" picks the band kernel for this state size."""
     return (batch > 0 and batch % 4 == 0
             and n_neurons * band_tile_columns(batch) * 4 >= BAND_AUTO_MIN_TILE_BYTES)
+
+
+# Fewest gathered state values (edges times columns) for which a recorded tick
+# copies a state that is not neuron-major into that layout first.  N=50k, M=1M,
+# B=8 (8M): the forward takes 41 us on a row-major state and 14 on a copy, the
+# weight gradient 37 and 9; the copy takes 4 us on the GPU and 6 on the host.
+RELAYOUT_MIN_GATHERS = 2_000_000
 
 
 class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
@@ -377,6 +405,7 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
         self.indexed_first_tick = True
         self._indexed_key = self._indexed_source = self._indexed_struct = None
         self._recorded_key, self._recorded_source, self._recorded_seen = None, None, 0
+        self._recorded_before = 0     # recorded ticks of the weight version before
         # The backward's transposed product on panels (False: the out-edge walk).
         self.transposed_panels_enabled = True
         self._transposed: TransposedPanels | None = None
@@ -402,16 +431,20 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
         (an optimizer step every tick) costs no slot-order copy.  From the
         second recorded tick of one version on (backpropagation through time,
         repeated evaluation) the panel kernel runs on a slot-order copy of that
-        version, built once.  A version is (tensor, in-place version counter),
-        so an update of the weights is never missed.
+        version, built once; when the version before saw two or more ticks (a
+        training loop through several), the copy is built for the first already
+        (N=166k, M=25M, two ticks: copy 65 + 2 x 33 us against indexed 80, copy
+        65 and 33).  A version is (tensor, in-place version counter), so an
+        update of the weights is never missed.
         """
         if self._panels is None:
             return None
         key = ("recorded",) + _weight_key(weight)
         if key != self._recorded_key or self._recorded_source is not weight:
+            self._recorded_before = self._recorded_seen
             self._recorded_key, self._recorded_source, self._recorded_seen = key, weight, 0
         self._recorded_seen += 1
-        if self._recorded_seen < 2:
+        if self._recorded_seen < 2 and self._recorded_before < 2:
             return self._panels.indexed_plan_struct()
         return self._slot_plan(self._panels, key, weight.detach(), ())
 
@@ -585,8 +618,14 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
             tick = self._prepared_recorded = PreparedTick(
                 self.extension, self.state, params, topology.in_rowptr, topology.in_col,
                 weight, **extra)
-        info = (self.extension, topology, us, vs, tick, self.source_major_weights,
-                self._transposed_layout(), self._prepared_backward)
+        transposed = self._transposed_layout()
+        if transposed is not None and self.state.requires_grad:
+            transposed.expect(weight)
+        batch = self.state.shape[0]
+        by_neuron = (self._panels is None and batch > 1
+                     and topology.n_edges * batch >= RELAYOUT_MIN_GATHERS)
+        info = (self.extension, topology, us, vs, tick, self.source_major_weights, transposed,
+                self._prepared_backward, by_neuron)
         self.state, self.dendritic_state, self.adaptation_state = _NativeTick.apply(
             info, self.state, self.dendritic_state, self.adaptation_state, weight, u, v,
             *params)

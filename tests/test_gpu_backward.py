@@ -311,3 +311,53 @@ def test_forward_of_a_recorded_tick_equals_the_inference_tick(gpu):
     assert recorded.last_backend == "native-autograd"
     assert torch.equal(plain.state, recorded.state.detach())
     assert torch.equal(plain.dendritic_state, recorded.dendritic_state.detach())
+
+
+@pytest.mark.parametrize("n,m,batch", [
+    (5, 12, 1), (300, 200, 2), (300, 900, 3), (257, 4000, 4), (130, 9000, 5), (200, 4000, 8),
+    (64, 3000, 12), (100, 2000, 16), (90, 1500, 17), (80, 1600, 20)])
+def test_edge_kernels_at_every_batch_form(gpu, n, m, batch):
+    """The backward's edge kernels take whole neuron-major rows (batch 2 or a multiple
+    of 4) or one column per lane, in lane groups sized to the mean degree: two ticks,
+    so the second's state is neuron-major and the first's is not, from fewer than one
+    edge per row to more than a wavefront's worth."""
+    print(f"case backward forms n={n} m={m} batch={batch}", flush=True)
+    g = graph(n, m, 31 + batch)
+    inputs = inputs_for(g, batch, 70 + batch)
+    kw = dict(scalar_drives=False, expanded=False)
+    native, _ = run(NativeDendriticMatrixRuntime, g, inputs, torch.float32, gpu, 2, **kw)
+    compare(native, oracle_gradients(g, inputs, 2, **kw))
+
+
+@pytest.mark.parametrize("batch,kernel,walk", [(1, "panels", False), (2, "rows", True),
+                                               (8, "rows", True)])
+def test_start_state_without_gradient_changes_no_other_gradient(gpu, monkeypatch, batch, kernel,
+                                                                walk):
+    """A start state that needs no gradient leaves out the first tick's transposed
+    product; with it (and with a row-major state copied to neuron-major first) the
+    other gradients are bitwise the same."""
+    print(f"case backward start state batch={batch} kernel={kernel}", flush=True)
+    from neurosim_gpu import native_compartmental as nc
+
+    g = graph(1500, 30_000, 4)
+    inputs = inputs_for(g, batch, 90 + batch)
+    results = {}
+    for mode in ("full", "leaf", "copied"):
+        monkeypatch.setattr(nc, "RELAYOUT_MIN_GATHERS", 0 if mode == "copied" else 1 << 60)
+        topo = topology(g, torch.float32, gpu)
+        topo.in_weight.requires_grad_(True)
+        mdl = model(inputs["params"], torch.float32, gpu, False)
+        state0 = leaf(inputs["state"], torch.float32, gpu)
+        rt = NativeDendriticMatrixRuntime(topo, mdl, state0.detach(), kernel=kernel)
+        rt.state = state0 if mode == "full" else state0.detach()
+        rt.step(0.2, dendritic_drive=0.1)
+        rt.step(0.3, dendritic_drive=0.1)
+        (rt.state * rt.state).sum().backward()
+        results[mode] = [topo.in_weight.grad, *(p.grad for p in params_of(mdl))]
+        if mode != "full":
+            assert (rt.source_major_weights._seen if walk else rt._transposed._seen) == 1
+    # The copied state is read whole rows at a time, so its weight gradient may sum the
+    # columns in another order: at most a few units in the last place of the terms.
+    for a, b, c in zip(*(results[m] for m in ("full", "leaf", "copied"))):
+        assert torch.equal(a, b)
+        assert float((a - c).abs().max()) <= batch * 2.0 ** -22 * float(a.abs().max())
