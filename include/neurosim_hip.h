@@ -371,6 +371,10 @@ typedef struct ns_step_grad_args {
  * (its recorded state needs none), so the transposed product W^T @ g is not
  * run; `d_state` is still required and receives the update's own part only. */
 #define NS_GRAD_NO_STATE 1
+/* ns_step_grad_args flags: `d_weight`, or every given `d_params` vector, already
+ * holds gradients of later ticks, and this tick's are added to them. */
+#define NS_GRAD_ADD_WEIGHT 2
+#define NS_GRAD_ADD_PARAMS 4
 
 /* Arguments of one weight encoding (fp8 e4m3 or NVFP4 CSR payload). */
 typedef struct ns_encode_args {

@@ -42,6 +42,7 @@ struct GradArgs {
   OutPlane gs, gd, ga, gu, gv;
   float* gj;             // [N][B]
   float* gp[6];
+  int32_t add_params;    // add to gp instead of storing
 };
 
 // One lane per (neuron, column), LB lanes per neuron; lane q takes columns q,
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(kGradThreads) void advance_backward_kernel(GradArgs
   }
 #pragma unroll
   for (int i = 0; i < 6; ++i)
-    if (q == 0 && A.gp[i]) A.gp[i][n] = sums[i];
+    if (q == 0 && A.gp[i]) A.gp[i][n] = A.add_params ? A.gp[i][n] + sums[i] : sums[i];
 }
 
 // The two edge kernels below give each row (a source, or a destination) a
@@ -182,12 +183,12 @@ __global__ __launch_bounds__(kGradThreads) void transposed_product_kernel(
 }
 
 // gw[e] = sum over columns b of gj[row, b] * s[b, col[e]], for the edges e of
-// each destination row: each lane sums its columns in order, the LPE lanes of
-// an edge by an xor butterfly.
+// each destination row (added to gw[e] when `add` is set): each lane sums its
+// columns in order, the LPE lanes of an edge by an xor butterfly.
 template <int VL, int LPE>
 __global__ __launch_bounds__(kGradThreads) void weight_gradient_kernel(
     const int32_t* rowptr, const int32_t* col, const float* gj, Plane s, int64_t N, int64_t B,
-    float* gw, int edge_lanes_log2) {
+    float* gw, int add, int edge_lanes_log2) {
   constexpr int kCols = VL * LPE;
   const int edge_lanes = 1 << edge_lanes_log2;
   const int group = LPE << edge_lanes_log2;
@@ -203,7 +204,11 @@ __global__ __launch_bounds__(kGradThreads) void weight_gradient_kernel(
     int64_t c[kGradUnroll];
 #pragma unroll
     for (int u = 0; u < kGradUnroll; ++u) c[u] = col[min(e + edge_lanes * u, e1 - 1)];
-    float sum[kGradUnroll];
+    float sum[kGradUnroll], before[kGradUnroll];
+    if (add && q == 0) {
+#pragma unroll
+      for (int u = 0; u < kGradUnroll; ++u) before[u] = gw[min(e + edge_lanes * u, e1 - 1)];
+    }
 #pragma unroll
     for (int u = 0; u < kGradUnroll; ++u) sum[u] = 0.0f;
     for (int64_t b0 = 0; b0 < B; b0 += kCols) {
@@ -230,7 +235,8 @@ __global__ __launch_bounds__(kGradThreads) void weight_gradient_kernel(
     }
 #pragma unroll
     for (int u = 0; u < kGradUnroll; ++u)
-      if (q == 0 && e + edge_lanes * u < e1) gw[e + edge_lanes * u] = sum[u];
+      if (q == 0 && e + edge_lanes * u < e1)
+        gw[e + edge_lanes * u] = add ? before[u] + sum[u] : sum[u];
   }
 }
 
@@ -310,7 +316,7 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
     return fail("the source-major view (out_rowptr, dst, out_weight_index) is required");
   if (!a.workspace) return fail("a workspace of 2*B*N floats is required");
   if (a.transposed_panels && batch > 2) return fail("transposed panels need batch 1 or 2");
-  if (a.flags & ~NS_GRAD_NO_STATE) return fail("unknown backward flags %d", a.flags);
+  if (a.flags & ~(NS_GRAD_NO_STATE | NS_GRAD_ADD_WEIGHT | NS_GRAD_ADD_PARAMS)) return fail("unknown backward flags %d", a.flags);
   const bool want_state = (a.flags & NS_GRAD_NO_STATE) == 0;
   const Extent outs[5] = {extent(a.d_state, batch, n), extent(a.d_dendrite, batch, n),
                           extent(a.d_adaptation, batch, n), extent(a.d_drive, batch, n),
@@ -356,6 +362,7 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
   G.gu = out_plane(a.d_drive); G.gv = out_plane(a.d_dendritic_drive);
   G.gj = gj;
   for (int i = 0; i < 6; ++i) G.gp[i] = a.d_params[i];
+  G.add_params = (a.flags & NS_GRAD_ADD_PARAMS) != 0;
   // The transposed product on panels: W^T @ gj added into d_state.
   ns_step_args transposed{};
   if (want_state && a.transposed_panels && a.matrix.n_edges > 0) {
@@ -412,7 +419,7 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
       with_edge_form(form, [&](auto vl, auto lpe) {
         weight_gradient_kernel<vl(), lpe()><<<lanes_grid(n, form.lpe << lg), kGradThreads, 0, s>>>(
             a.matrix.rowptr, a.matrix.col, gj, plane(a.state, a.state.data), n, batch, a.d_weight,
-            lg);
+            (a.flags & NS_GRAD_ADD_WEIGHT) != 0, lg);
       });
     }
   }

@@ -141,7 +141,7 @@ class _StepGradArgs(ctypes.Structure):
                 ("current", _c_ptr), ("out_weight", _c_ptr), ("transposed_panels", _c_ptr),
                 ("flags", ctypes.c_int32), ("reserved", ctypes.c_int32)]
 
-GRAD_NO_STATE = 1        # NS_GRAD_NO_STATE
+GRAD_NO_STATE, GRAD_ADD_WEIGHT, GRAD_ADD_PARAMS = 1, 2, 4   # NS_GRAD_*
 
 
 class _EncodeArgs(ctypes.Structure):
@@ -1289,7 +1289,11 @@ class PreparedBackward:
     workspace (one allocation), writes the per-call words and launches.  The
     results equal ``NativeExtension.dendritic_step_backward`` on the same inputs.
     ``need_state=False`` leaves out the transposed product: the returned d_state
-    is then the update's own part, for a caller that drops it."""
+    is then the update's own part, for a caller that drops it.  ``sums`` gives the
+    weight gradient and the parameter gradients' block of later ticks, which this
+    tick's are added to in place (as autograd would add them, in the same order).
+    Last of the results is the parameter gradients' block; ``split=False`` leaves
+    out the list of its rows."""
 
     def __init__(self, extension: "NativeExtension", state: torch.Tensor, params, rowptr, col,
                  weight, out_rowptr, dst, weight_index):
@@ -1333,7 +1337,7 @@ class PreparedBackward:
                  dendritic_scalar, grad_state, grad_dendrite, grad_adaptation, *,
                  need_drive=False, need_dendritic=False, need_weight=False,
                  need_params=(False,) * 6, out_weight=None, current=None,
-                 transposed_panels=None, need_state=True):
+                 transposed_panels=None, need_state=True, sums=(None, None), split=True):
         _check_state(state)
         if state.device != self.device:
             raise RuntimeError("all tensors must be on the state's CUDA device")
@@ -1372,27 +1376,47 @@ class PreparedBackward:
             words += (base + index * size, 1, batch) if present else (0, 0, 0)
         _OUTS5.pack_into(args, _GRAD_OUT, *words)
         planes = storage.transpose(1, 2).unbind(0)
-        d_weight = torch.empty_like(weight) if need_weight else None
+        # Sums of later ticks' gradients are added to in place.
+        d_weight, block = sums
+        flags = 0 if need_state else GRAD_NO_STATE
+        if d_weight is not None:
+            _check_float(d_weight, state, "weight gradient")
+            if d_weight.shape != weight.shape or not d_weight.is_contiguous():
+                raise RuntimeError("the weight gradient must be a contiguous [M] vector")
+            flags |= GRAD_ADD_WEIGHT
+        elif need_weight:
+            d_weight = torch.empty(weight.shape, dtype=torch.float32, device=self.device)
         wanted = [i for i, want in enumerate(need_params) if want]
-        work = self._work               # first in the block, so 16-byte aligned
-        block = torch.empty(work + len(wanted) * n, dtype=torch.float32, device=self.device)
-        d_params = [None] * 6
+        work = self._work
+        if block is not None:
+            _check_float(block, state, "parameter gradients")
+            if block.shape != (len(wanted) * n,) or not block.is_contiguous():
+                raise RuntimeError("the parameter gradients must be one contiguous vector")
+            flags |= GRAD_ADD_PARAMS
+            workspace = torch.empty(work, dtype=torch.float32, device=self.device)
+            start = block.data_ptr()
+        else:                           # the workspace first, so that it is 16-byte aligned
+            workspace = torch.empty(work + len(wanted) * n, dtype=torch.float32,
+                                    device=self.device)
+            start = workspace.data_ptr() + 4 * work
+            block = workspace[work:] if wanted else None
         param_ptrs = [0] * 6
         for k, i in enumerate(wanted):
-            d_params[i] = block[work + k * n:work + (k + 1) * n]
-            param_ptrs[i] = d_params[i].data_ptr()
-        workspace_ptr = block.data_ptr() if work else 0
+            param_ptrs[i] = start + 4 * k * n
         _POINTERS11.pack_into(args, _GRAD_POINTERS,
                               d_weight.data_ptr() if d_weight is not None and weight.numel() else 0,
-                              *param_ptrs, workspace_ptr, current_ptr, out_weight_ptr,
+                              *param_ptrs, workspace.data_ptr() if work else 0, current_ptr,
+                              out_weight_ptr,
                               ctypes.addressof(transposed_panels) if transposed_panels is not None
                               else 0)
-        args.flags = 0 if need_state else GRAD_NO_STATE
+        args.flags = flags
         _raise_on(self.lib.ns_dendritic_step_backward(self._ref, current_stream(self.device)),
                   self.lib)
         d_drive = planes[3] if need_drive else None
         d_dendritic = planes[count - 1] if need_dendritic else None
-        return (planes[0], planes[1], planes[2], d_drive, d_dendritic, d_weight, d_params)
+        rows = iter(block.view(-1, n).unbind(0)) if split and block is not None else None
+        d_params = [next(rows) if rows is not None and want else None for want in need_params]
+        return (planes[0], planes[1], planes[2], d_drive, d_dendritic, d_weight, d_params, block)
 
 
 class PreparedEvent:

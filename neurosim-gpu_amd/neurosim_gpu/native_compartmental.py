@@ -24,6 +24,8 @@ library raises at construction, nothing falls back silently.
 from __future__ import annotations
 
 import warnings
+import weakref
+from operator import is_
 from types import SimpleNamespace
 
 import torch
@@ -31,7 +33,7 @@ import torch
 from .compartmental import DendriticDynamics, DendriticMatrixRuntime, DendriticPELSRuntime
 from .native import (BAND_WIDTH, EVENT_ACTIVITY_SLOTS, EVENT_ACTIVITY_STRIDE, BandLayout,
                      NativeExtension, PanelLayout, PreparedAccumulate, PreparedBackward,
-                     PreparedEvent, PreparedTick, _neuron_major, encode_weights,
+                     PreparedEvent, PreparedTick, _neuron_major, current_stream, encode_weights,
                      load_native_extension, new_planes, panel_geometry)
 from .topology import SparseTopology
 
@@ -61,6 +63,7 @@ class _NativeCompartments:
         # The backward's prepared launch, shared by the ticks recorded here (a
         # one-element holder, since the backward runs after the forward returns).
         self._prepared_backward = [None]
+        self._recording = None      # the run of recorded ticks (_Recording)
 
     def _parameters(self) -> list[torch.Tensor]:
         model = self.compartment_dynamics
@@ -204,35 +207,83 @@ class TransposedPanels:
         return self.layout.plan_struct(slots, None)
 
 
+class _TickInfo:
+    """What one recorded tick needs besides its tensors."""
+
+    __slots__ = ("extension", "topology", "us", "vs", "tick", "source_major", "transposed",
+                 "prepared", "by_neuron", "weight", "params", "first")
+
+    def __init__(self, **fields) -> None:
+        for name, value in fields.items():
+            setattr(self, name, value)
+
+
+class _Recording:
+    """A run of recorded ticks, each starting from the states the one before
+    returned, on the same weights and parameters.
+
+    Only its first tick takes the weights and parameters as autograd inputs.
+    Every tick also returns two tokens, zero-stride tensors of the shapes of the
+    weight gradient and of the parameter gradients' block, and takes those of the
+    tick before.  The gradient of a token is the sum of the later ticks'
+    gradients, which a tick's backward adds its own to in place and hands on, so
+    a backward through T ticks adds no pair of gradients outside the kernels
+    (seven torch additions per tick otherwise).  The states are held weakly:
+    once the caller drops them the tokens, and the graph behind them, go too."""
+
+    __slots__ = ("states", "weight", "params", "versions", "topology", "stream", "tokens")
+
+    def __init__(self, states, weight, params, versions, topology, stream, tokens) -> None:
+        self.weight, self.params, self.topology, self.stream = weight, params, topology, stream
+        self.versions, self.tokens = versions, tokens
+        self.states = (weakref.ref(states[0], self._drop), *map(weakref.ref, states[1:]))
+
+    def _drop(self, _) -> None:
+        self.tokens = None
+
+    def continues(self, states, weight, params, versions, topology, stream) -> bool:
+        return (self.tokens is not None and topology is self.topology
+                and all(ref() is s for ref, s in zip(self.states, states))
+                and weight is self.weight and all(map(is_, params, self.params))
+                and stream == self.stream and versions == self.versions)
+
+
 class _NativeTick(torch.autograd.Function):
     """One float32 fused tick (ns_dendritic_step) whose backward is native too
     (ns_dendritic_step_backward): gradients of the states, tensor drives, the
     six parameter vectors and the CSR weights, as autograd through the
-    reference's torch step would give them."""
+    reference's torch step would give them.  The weights and parameters are
+    inputs of the first tick of a ``_Recording``; later ticks get the tokens of
+    the tick before in their place."""
 
     @staticmethod
-    def forward(ctx, info, state, dendrite, adaptation, weight, drive, dendritic_drive, *params):
-        _, _, us, vs, tick, _, _, _, by_neuron = info
-        if by_neuron and not _neuron_major(state):
+    def forward(ctx, info, state, dendrite, adaptation, drive, dendritic_drive, *linked):
+        if info.by_neuron and not _neuron_major(state):
             # One gathered run per edge for the forward and the weight gradient.
             state = new_planes(1, *state.shape, state)[0].copy_(state)
         # The launch arguments were prepared (and validated) for this weight, plan
         # and these parameters; j = W @ s is kept for the backward, which then
         # needs no product of its own.
-        *outs, current = tick(state, dendrite, adaptation, drive, us, dendritic_drive, vs,
-                              current=True)
+        *outs, current = info.tick(state, dendrite, adaptation, drive, info.us, dendritic_drive,
+                                   info.vs, current=True)
         ctx.current = current
         ctx.info = info
         ctx.has_drive = (drive is not None, dendritic_drive is not None)
+        weight, params = info.weight, info.params
         saved = [state, dendrite, adaptation, weight, *params]
         saved += [t for t in (drive, dendritic_drive) if t is not None]
         ctx.save_for_backward(*saved)
         ctx.set_materialize_grads(False)
-        return tuple(outs)
+        ctx.wants = (weight.requires_grad, tuple(p.requires_grad for p in params))
+        zero = state.new_empty(1)
+        tokens = (zero.expand(weight.numel()) if ctx.wants[0] else None,
+                  zero.expand(sum(ctx.wants[1]) * state.shape[1]) if any(ctx.wants[1]) else None)
+        return (*outs, *tokens)
 
     @staticmethod
-    def backward(ctx, grad_state, grad_dendrite, grad_adaptation):
-        extension, topology, us, vs, _, source_major, transposed, cache, _ = ctx.info
+    def backward(ctx, grad_state, grad_dendrite, grad_adaptation, sum_weight, sum_params):
+        info = ctx.info
+        topology = info.topology
         saved = list(ctx.saved_tensors)
         state, dendrite, adaptation, weight = saved[:4]
         params = saved[4:10]
@@ -240,28 +291,30 @@ class _NativeTick(torch.autograd.Function):
         drive = next(rest) if ctx.has_drive[0] else None
         dendritic_drive = next(rest) if ctx.has_drive[1] else None
         needs = ctx.needs_input_grad
+        need_weight, need_params = ctx.wants
         # A start state that needs no gradient needs no transposed product either.
         panels = out_weight = None
         if needs[1]:
-            panels = transposed.plan(weight) if transposed is not None else None
+            panels = info.transposed.plan(weight) if info.transposed is not None else None
             out_weight = (None if panels is not None
-                          else source_major.get(weight, topology.out_weight_index))
+                          else info.source_major.get(weight, topology.out_weight_index))
         fixed = (topology.in_rowptr, topology.in_col, weight, topology.out_rowptr,
                  topology.dst, topology.out_weight_index)
+        cache = info.prepared
         prepared = cache[0]
         if prepared is None or not prepared.matches(state, params, *fixed):
-            prepared = cache[0] = PreparedBackward(extension, state, params, *fixed)
-        (d_state, d_dendrite, d_adaptation, d_drive, d_dendritic, d_weight,
-         d_params) = prepared(
-            state, dendrite, adaptation, drive, us, dendritic_drive, vs, grad_state,
-            grad_dendrite, grad_adaptation, need_drive=bool(needs[5]),
-            need_dendritic=bool(needs[6]), need_weight=bool(needs[4]),
-            need_params=tuple(bool(x) for x in needs[7:13]),
+            prepared = cache[0] = PreparedBackward(info.extension, state, params, *fixed)
+        (d_state, d_dendrite, d_adaptation, d_drive, d_dendritic, d_weight, d_params,
+         block) = prepared(
+            state, dendrite, adaptation, drive, info.us, dendritic_drive, info.vs, grad_state,
+            grad_dendrite, grad_adaptation, need_drive=bool(needs[4]),
+            need_dendritic=bool(needs[5]), need_weight=need_weight, need_params=need_params,
             out_weight=out_weight, current=ctx.current, transposed_panels=panels,
-            need_state=bool(needs[1]))
+            need_state=bool(needs[1]), sums=(sum_weight, sum_params), split=info.first)
         ctx.current = None
+        linked = (d_weight, *d_params) if info.first else (d_weight, block)
         return (None, d_state if needs[1] else None, d_dendrite if needs[2] else None,
-                d_adaptation if needs[3] else None, d_weight, d_drive, d_dendritic, *d_params)
+                d_adaptation if needs[3] else None, d_drive, d_dendritic, *linked)
 
 
 # "auto" takes column panels (batch 1-2) when the graph has at least
@@ -624,11 +677,21 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
         batch = self.state.shape[0]
         by_neuron = (self._panels is None and batch > 1
                      and topology.n_edges * batch >= RELAYOUT_MIN_GATHERS)
-        info = (self.extension, topology, us, vs, tick, self.source_major_weights, transposed,
-                self._prepared_backward, by_neuron)
-        self.state, self.dendritic_state, self.adaptation_state = _NativeTick.apply(
-            info, self.state, self.dendritic_state, self.adaptation_state, weight, u, v,
-            *params)
+        states = (self.state, self.dendritic_state, self.adaptation_state)
+        stream = current_stream(self.state.device)
+        recording = self._recording
+        versions = [(t._version, t.requires_grad) for t in (weight, *params)]
+        first = recording is None or not recording.continues(states, weight, params, versions,
+                                                             topology, stream)
+        info = _TickInfo(extension=self.extension, topology=topology, us=us, vs=vs, tick=tick,
+                         source_major=self.source_major_weights, transposed=transposed,
+                         prepared=self._prepared_backward, by_neuron=by_neuron, weight=weight,
+                         params=params, first=first)
+        linked = (weight, *params) if first else recording.tokens
+        *states, token_weight, token_params = _NativeTick.apply(info, *states, u, v, *linked)
+        self._recording = _Recording(states, weight, params, versions, topology, stream,
+                                     (token_weight, token_params))
+        self.state, self.dendritic_state, self.adaptation_state = states
         self.last_backend = "native-autograd"
         return self.state
 

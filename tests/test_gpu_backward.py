@@ -361,3 +361,84 @@ def test_start_state_without_gradient_changes_no_other_gradient(gpu, monkeypatch
     for a, b, c in zip(*(results[m] for m in ("full", "leaf", "copied"))):
         assert torch.equal(a, b)
         assert float((a - c).abs().max()) <= batch * 2.0 ** -22 * float(a.abs().max())
+
+
+@pytest.mark.parametrize("batch,kernel", [(1, "panels"), (3, "rows"), (8, "rows")])
+def test_gradients_summed_through_the_ticks_equal_separate_ones(gpu, batch, kernel):
+    """A run of recorded ticks hands its weight and parameter gradients from tick to
+    tick, each backward adding to them in place.  Against ticks recorded one by one
+    (autograd adds their gradients, in the same order): bitwise, also through a second
+    backward of the same graph, with some parameters frozen, and for a loss that leaves
+    out the last ticks."""
+    print(f"case backward linked ticks batch={batch} kernel={kernel}", flush=True)
+    g = graph(900, 20_000, 8)
+    inputs = inputs_for(g, batch, 50 + batch)
+
+    def gradients(linked: bool, frozen: bool, early: bool):
+        topo = topology(g, torch.float32, gpu)
+        topo.in_weight.requires_grad_(True)
+        mdl = model(inputs["params"], torch.float32, gpu, False)
+        if frozen:
+            mdl.soma.gain.requires_grad_(False)
+            mdl.coupling.requires_grad_(False)
+        rt = NativeDendriticMatrixRuntime(topo, mdl, torch.full((batch, 900), .3, device=gpu),
+                                          kernel=kernel)
+        states = []
+        for t in range(4):
+            rt.step(0.1 * t, dendritic_drive=0.1)
+            states.append(rt.state)
+            if not linked:
+                rt._recording = None
+        loss = (states[1 if early else 3] ** 2).sum() + (states[1] * 0.5).sum()
+        wanted = [topo.in_weight, *(p for p in params_of(mdl) if p.requires_grad)]
+        first = torch.autograd.grad(loss, wanted, retain_graph=True)
+        second = torch.autograd.grad(loss, wanted)
+        return first, second
+
+    for frozen in (False, True):
+        for early in (False, True):
+            one, again = gradients(True, frozen, early)
+            separate, _ = gradients(False, frozen, early)
+            for a, b, c in zip(one, separate, again):
+                assert torch.equal(a, b)
+                # the second backward recomputes j = W @ s on row blocks
+                assert float((a - c).abs().max()) <= 1e-5 * float(a.abs().max())
+
+
+def test_a_run_of_recorded_ticks_ends_where_its_inputs_change(gpu):
+    """Detached states, restored states, an in-place update and a newly trained
+    parameter each start a new run; gradients then match ticks recorded one by one."""
+    print("case backward run boundaries", flush=True)
+    g = graph(500, 6_000, 2)
+    inputs = inputs_for(g, 2, 12)
+
+    def gradients(linked: bool):
+        topo = topology(g, torch.float32, gpu)
+        topo.in_weight.requires_grad_(True)
+        mdl = model(inputs["params"], torch.float32, gpu, False)
+        mdl.coupling.requires_grad_(False)
+        rt = NativeDendriticMatrixRuntime(topo, mdl, torch.full((2, 500), .3, device=gpu))
+
+        def step(u):
+            rt.step(u, dendritic_drive=0.1)
+            if not linked:
+                rt._recording = None
+
+        step(0.1)
+        step(0.2)
+        kept = (rt.state, rt.dendritic_state, rt.adaptation_state)
+        step(0.3)
+        loss = rt.state.sum()
+        rt.state, rt.dendritic_state, rt.adaptation_state = kept    # a second branch
+        mdl.coupling.requires_grad_(True)
+        step(0.4)
+        step(0.1)
+        loss = loss + (rt.state * 2).sum()
+        rt.state = rt.state.detach()                                # truncated
+        step(0.2)
+        loss = loss + (rt.state ** 2).sum()
+        return torch.autograd.grad(loss, [topo.in_weight, *params_of(mdl)])
+
+    for a, b in zip(gradients(True), gradients(False)):
+        # branches meet in another order of additions: a few roundings of the sum
+        assert float((a - b).abs().max()) <= 2.0 ** -20 * float(b.abs().max())
