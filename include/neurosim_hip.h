@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define NS_ABI_VERSION 20
+#define NS_ABI_VERSION 21
 
 /* Return codes. */
 #define NS_OK 0
@@ -287,6 +287,13 @@ typedef struct ns_event_args {
      active out-edges, the reference's PELS policy measure (runtime.py:129-165).
      The caller zeroes and reads them (NULL: not counted). */
   int64_t* activity;
+  /* NS_EVENT_PRODUCT only: the destination-major view (rowptr [N+1], source of
+     each CSR edge [M]; `weight` are its weights), and optionally a workspace of
+     ceil(B*N / 64) words, overwritten, in which the advance marks the pairs that
+     emit (bit n*B + b), so that the product skips the others' edges. */
+  const int32_t* in_rowptr;
+  const int32_t* in_col;
+  uint64_t* emitting;
 } ns_event_args;
 
 #define NS_EVENT_ACTIVITY_SLOTS 32
@@ -299,6 +306,10 @@ typedef struct ns_event_args {
  * propagation of emitted deltas (runtime.py:233-235), which beats the scatter
  * when many sources emit. */
 #define NS_EVENT_ADVANCE_ONLY 1
+/* With NS_EVENT_ADVANCE_ONLY and pending_in: a second launch adds W @ delta into
+ * `current`, each destination's in-edges summed by one group of lanes, no atomics
+ * (pairs with a zero delta contribute nothing, as in the scatter). */
+#define NS_EVENT_PRODUCT 4
 
 /* Arguments of a plain CSR product J = W @ S (no neuron update). */
 typedef struct ns_spmm_args {

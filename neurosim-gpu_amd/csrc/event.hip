@@ -28,6 +28,7 @@
 #include <algorithm>
 
 #include "ns_common.h"
+#include "ns_edge_rows.h"
 #include "ns_host.h"
 
 namespace ns {
@@ -49,6 +50,9 @@ struct EventArgs {
   float* pending_in;
   float* pending_out;
   unsigned long long* activity;
+  const int32_t* in_rowptr;
+  const int32_t* in_col;
+  unsigned long long* emitting;
   int32_t column_log2;  // log2 B when B is a power of two in [2, 64], else 0
 };
 
@@ -331,8 +335,127 @@ __global__ __launch_bounds__(kThreads) void event_tick_kernel(EventArgs A) {
     dl = advance_loaded_pair(A, n, b, j, in, active);
     if constexpr (!kScatter) A.delta[i] = dl;
   }
+  if constexpr (!kScatter) {
+    if (A.emitting) {
+      const unsigned long long word = __ballot(dl != 0.0f);
+      if (lane == 0 && i < A.count) A.emitting[chunk] = word;
+    }
+  }
   if constexpr (kCount) count_activity(A, active ? end - start : 0);
   if constexpr (kScatter) scatter_wave(A, chunk, lane, dl, start, end, A.pending_out, 1, A.B);
+}
+
+// current[b, n] += sum over in-edges e of destination n of weight[e] *
+// delta[in_col[e], b], the pairs that emitted nothing left out (a scatter pushes
+// nothing for them, whatever the weight).  Lane groups as in ns_edge_rows.h, and
+// at most kProductBlocks workgroups that walk the rows.  kBits (batch 1 or 2): the
+// emitting pairs' bitmap is staged in LDS first, and an edge whose source is
+// silent costs its column index and one LDS read: a stream of 4 bytes per edge
+// with gathers for the active ones only, where the unpruned product is bound by
+// one L2 request per edge.
+constexpr int kProductThreads = 512;
+constexpr int kProductBlocks = 1024;
+constexpr int64_t kProductBitBytes = 64 * 1024;  // largest bitmap staged
+
+template <int VL, int LPE, bool kBits>
+__global__ __launch_bounds__(kProductThreads) void event_product_kernel(EventArgs A,
+                                                                        int edge_lanes_log2) {
+  extern __shared__ unsigned long long staged[];
+  const int64_t words = (A.count + 63) / 64;
+  if constexpr (kBits) {
+    for (int64_t i = threadIdx.x; i < words; i += kProductThreads) staged[i] = A.emitting[i];
+    __syncthreads();
+  }
+  const uint32_t* const bits = reinterpret_cast<const uint32_t*>(staged);
+  constexpr int kCols = VL * LPE;
+  const int edge_lanes = 1 << edge_lanes_log2;
+  const int group = LPE << edge_lanes_log2;
+  const int group_log2 = __builtin_ctz(LPE) + edge_lanes_log2;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kProductThreads + threadIdx.x;
+  const int64_t step = (static_cast<int64_t>(gridDim.x) * kProductThreads) >> group_log2;
+  const int lane = static_cast<int>(t & (group - 1));
+  const int q = lane & (LPE - 1), el = lane / LPE;
+  const int64_t B = A.B;
+  for (int64_t n = t >> group_log2; n < A.N; n += step) {
+    const int32_t e0 = A.in_rowptr[n], e1 = A.in_rowptr[n + 1];
+    for (int64_t b0 = 0; b0 < B; b0 += kCols) {
+      const int64_t b = b0 + q * VL;
+      const bool have = b < B;
+      float acc[VL];
+#pragma unroll
+      for (int k = 0; k < VL; ++k) acc[k] = 0.0f;
+      for (int32_t e = e0 + el; e < e1; e += edge_lanes * kEdgeUnroll) {
+        int32_t c[kEdgeUnroll];
+        float w[kEdgeUnroll], x[kEdgeUnroll][VL];
+#pragma unroll
+        for (int u = 0; u < kEdgeUnroll; ++u) {
+          const int32_t at = min(e + edge_lanes * u, e1 - 1);
+          c[u] = A.in_col[at];
+          if constexpr (!kBits) w[u] = A.weight[at];
+        }
+#pragma unroll
+        for (int u = 0; u < kEdgeUnroll; ++u) {
+          const int32_t at = e + edge_lanes * u;
+          if constexpr (kBits) {
+            // Batch 1 or 2: the source's bits lie in one word, at c * B.
+            const uint32_t bit = static_cast<uint32_t>(c[u]) * VL;
+            const uint32_t word = bits[bit >> 5] >> (bit & 31);
+            w[u] = 0.0f;
+#pragma unroll
+            for (int k = 0; k < VL; ++k) x[u][k] = 0.0f;
+            if (at < e1 && (word & ((1u << VL) - 1)) != 0) {
+              w[u] = A.weight[at];
+              load_row<VL>(A.delta + static_cast<int64_t>(c[u]) * B, x[u]);
+            }
+          } else {
+            load_row<VL>(A.delta + static_cast<int64_t>(c[u]) * B + (have ? b : 0), x[u]);
+#pragma unroll
+            for (int k = 0; k < VL; ++k) x[u][k] = at < e1 ? x[u][k] : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kEdgeUnroll; ++u) {
+#pragma unroll
+          for (int k = 0; k < VL; ++k)
+            acc[k] = x[u][k] != 0.0f ? __builtin_fmaf(w[u], x[u][k], acc[k]) : acc[k];
+        }
+      }
+      for (int off = LPE; off < group; off <<= 1) {
+#pragma unroll
+        for (int k = 0; k < VL; ++k) acc[k] += __shfl_xor(acc[k], off, 64);
+      }
+      if (el == 0 && have) {
+#pragma unroll
+        for (int k = 0; k < VL; ++k) {
+          float* const at = A.current + (b + k) * A.csb + n * A.csn;
+          *at = *at + acc[k];
+        }
+      }
+    }
+  }
+}
+
+hipError_t launch_product(const EventArgs& A, int64_t n_edges, hipStream_t s) {
+  const int64_t bit_bytes = (A.count + 63) / 64 * 8;
+  const bool aligned = reinterpret_cast<uintptr_t>(A.delta) % 16 == 0;
+  const bool pruned = A.emitting && bit_bytes <= kProductBitBytes &&
+                      (A.B == 1 || (A.B == 2 && aligned));
+  const EdgeForm form = edge_form(A.B, aligned);
+  const int lg = edge_lanes_for(n_edges, A.N, form.lpe);
+  const int64_t lanes = A.N * (form.lpe << lg);
+  const dim3 grid(static_cast<unsigned>(
+      std::min<int64_t>((lanes + kProductThreads - 1) / kProductThreads,
+                        pruned ? kProductBlocks : int64_t{1} << 20)));
+  if (pruned) {
+    const unsigned lds = static_cast<unsigned>(bit_bytes);
+    if (A.B == 1) event_product_kernel<1, 1, true><<<grid, kProductThreads, lds, s>>>(A, lg);
+    else event_product_kernel<2, 1, true><<<grid, kProductThreads, lds, s>>>(A, lg);
+  } else {
+    with_edge_form(form, [&](auto vl, auto lpe) {
+      event_product_kernel<vl(), lpe(), false><<<grid, kProductThreads, 0, s>>>(A, lg);
+    });
+  }
+  return hipGetLastError();
 }
 
 }  // namespace ns
@@ -368,8 +491,10 @@ extern "C" int ns_dendritic_event(const ns_event_args* args, void* stream) {
   if (!a.out_state.data || !a.out_dendrite.data || !a.out_adaptation.data ||
       !a.out_emitted.data)
     return fail("four output planes are required");
-  if (a.flags & ~NS_EVENT_ADVANCE_ONLY) return fail("unknown event flags %d", a.flags);
+  if (a.flags & ~(NS_EVENT_ADVANCE_ONLY | NS_EVENT_PRODUCT))
+    return fail("unknown event flags %d", a.flags);
   const bool advance_only = (a.flags & NS_EVENT_ADVANCE_ONLY) != 0;
+  const bool product = (a.flags & NS_EVENT_PRODUCT) != 0;
   // The one-launch forms read j = current + pending_in; the scattering one
   // also needs pending_out, the advance-only one writes `delta` instead.
   const bool fused = a.pending_in != nullptr;
@@ -380,12 +505,18 @@ extern "C" int ns_dendritic_event(const ns_event_args* args, void* stream) {
     if (fused != (a.pending_out != nullptr)) return fail("pending_in and pending_out go together");
     if (!fused && !a.delta) return fail("a delta workspace is required");
   }
+  if (product) {
+    if (!advance_only || !fused)
+      return fail("the product follows a fused advance-only tick (pending_in)");
+    if (a.n_edges > 0 && (!a.in_rowptr || !a.in_col))
+      return fail("the product needs in_rowptr and in_col");
+  }
   if (a.activity && !fused)
     return fail("activity counts need the one-launch tick (pending_in)");
   const int64_t B = a.batch, N = a.n_neurons;
   // Written memory: the four planes, then the workspaces (pending buffers and
   // delta, entry n*B + b) and the activity counters.
-  Extent outs[8] = {extent(a.out_state, B, N), extent(a.out_dendrite, B, N),
+  Extent outs[9] = {extent(a.out_state, B, N), extent(a.out_dendrite, B, N),
                     extent(a.out_adaptation, B, N), extent(a.out_emitted, B, N)};
   int n_outs = 4;
   if (a.pending_in) outs[n_outs++] = extent_of(a.pending_in, 1, B, B, N);
@@ -394,6 +525,8 @@ extern "C" int ns_dendritic_event(const ns_event_args* args, void* stream) {
   if (a.activity)
     outs[n_outs++] = extent_of(a.activity, 0, 1, 1,
                                2 * NS_EVENT_ACTIVITY_SLOTS * NS_EVENT_ACTIVITY_STRIDE);
+  if (product && a.emitting)
+    outs[n_outs++] = extent_of(a.emitting, 0, 1, 1, 2 * ((B * N + 63) / 64));
   const Extent ins[8] = {extent(a.state, B, N), extent(a.dendrite, B, N),
                          extent(a.adaptation, B, N), extent(a.drive, B, N),
                          extent(a.dendritic_drive, B, N), extent(a.emitted, B, N),
@@ -429,6 +562,8 @@ extern "C" int ns_dendritic_event(const ns_event_args* args, void* stream) {
   A.out_weight = a.out_weight;
   A.pending_in = a.pending_in; A.pending_out = a.pending_out;
   A.activity = reinterpret_cast<unsigned long long*>(a.activity);
+  A.in_rowptr = a.in_rowptr; A.in_col = a.in_col;
+  A.emitting = product ? reinterpret_cast<unsigned long long*>(a.emitting) : nullptr;
   // Column-grouped scatter for B = 2, 4, ..., 64 (a wavefront then holds whole sources).
   A.column_log2 = 0;
   for (int lg = 1; lg <= 6; ++lg)
@@ -444,8 +579,13 @@ extern "C" int ns_dendritic_event(const ns_event_args* args, void* stream) {
       if (A.activity) event_tick_kernel<true, true><<<grid, dim3(kThreads), 0, s>>>(A);
       else event_tick_kernel<true, false><<<grid, dim3(kThreads), 0, s>>>(A);
     }
-    const hipError_t err = hipGetLastError();
-    return err == hipSuccess ? NS_OK : fail_launch("event tick", err);
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return fail_launch("event tick", err);
+    if (product && a.n_edges > 0) {
+      err = launch_product(A, a.n_edges, s);
+      if (err != hipSuccess) return fail_launch("event product", err);
+    }
+    return NS_OK;
   }
   const int64_t advance_blocks = std::min<int64_t>((A.count + kThreads - 1) / kThreads, 65536);
   event_advance_kernel<<<dim3(static_cast<unsigned>(advance_blocks)), dim3(kThreads), 0, s>>>(A);

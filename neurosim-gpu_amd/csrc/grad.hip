@@ -22,17 +22,15 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <type_traits>
 
 #include "ns_common.h"
+#include "ns_edge_rows.h"
 #include "ns_host.h"
 
 namespace ns {
 namespace {
 
 constexpr int kGradThreads = 256;
-constexpr int kGradUnroll = 4;  // edges per lane per round of the edge loops
-
 struct GradArgs {
   int64_t N, B;
   Plane s, d, a, u, v;
@@ -105,27 +103,6 @@ __global__ __launch_bounds__(kGradThreads) void advance_backward_kernel(GradArgs
     if (q == 0 && A.gp[i]) A.gp[i][n] = A.add_params ? A.gp[i][n] + sums[i] : sums[i];
 }
 
-// The two edge kernels below give each row (a source, or a destination) a
-// power-of-two group of lanes: LPE lanes per edge, VL neighbouring columns each
-// (one 4 * VL byte load of a neuron-major row; VL = 1 takes any strides), and
-// `edge_lanes` edges at a time, kGradUnroll rounds of them in flight.  The host
-// picks edge_lanes so that a row of average length is about one round
-// (edge_lanes_for).  A wavefront per row, every lane walking its edge's columns
-// by itself, left two thirds of the lanes idle at 20 edges per row and read
-// each gathered row in 4-byte pieces.
-
-template <int VL>
-__device__ __forceinline__ void load_row(const float* at, float x[VL]) {
-  typedef float vec __attribute__((ext_vector_type(VL == 1 ? 2 : VL)));
-  if constexpr (VL == 1) {
-    x[0] = *at;
-  } else {
-    const vec y = *reinterpret_cast<const vec*>(at);
-#pragma unroll
-    for (int k = 0; k < VL; ++k) x[k] = y[k];
-  }
-}
-
 // gs[b, c] += sum over out-edges e of source c of w[owi[e]] * gj[dst[e], b].
 template <int VL, int LPE>
 __global__ __launch_bounds__(kGradThreads) void transposed_product_kernel(
@@ -149,20 +126,20 @@ __global__ __launch_bounds__(kGradThreads) void transposed_product_kernel(
     // Every load of a round is issued before the first multiply (an edge past
     // the row's end rereads the row's last edge and adds nothing), so a round
     // waits on memory twice: indices and weights, then the gathered rows.
-    for (int32_t e = e0 + el; e < e1; e += edge_lanes * kGradUnroll) {
-      float weight[kGradUnroll], g[kGradUnroll][VL];
-      int64_t to[kGradUnroll];
+    for (int32_t e = e0 + el; e < e1; e += edge_lanes * kEdgeUnroll) {
+      float weight[kEdgeUnroll], g[kEdgeUnroll][VL];
+      int64_t to[kEdgeUnroll];
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u) {
+      for (int u = 0; u < kEdgeUnroll; ++u) {
         const int32_t at = min(e + edge_lanes * u, e1 - 1);
         // Source-major weights stream; otherwise each one is a gather into the CSR order.
         weight[u] = w_out ? w_out[at] : w[owi[at]];
         to[u] = dst[at];
       }
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u) load_row<VL>(gj + to[u] * B + (have ? b : 0), g[u]);
+      for (int u = 0; u < kEdgeUnroll; ++u) load_row<VL>(gj + to[u] * B + (have ? b : 0), g[u]);
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u) {
+      for (int u = 0; u < kEdgeUnroll; ++u) {
         if (e + edge_lanes * u >= e1) break;
 #pragma unroll
         for (int k = 0; k < VL; ++k) acc[k] = __builtin_fmaf(weight[u], g[u][k], acc[k]);
@@ -200,29 +177,29 @@ __global__ __launch_bounds__(kGradThreads) void weight_gradient_kernel(
   const int32_t e0 = rowptr[r], e1 = rowptr[r + 1];
   // A round's column indices load together, then their state gathers, then the
   // stores.
-  for (int32_t e = e0 + el; e < e1; e += edge_lanes * kGradUnroll) {
-    int64_t c[kGradUnroll];
+  for (int32_t e = e0 + el; e < e1; e += edge_lanes * kEdgeUnroll) {
+    int64_t c[kEdgeUnroll];
 #pragma unroll
-    for (int u = 0; u < kGradUnroll; ++u) c[u] = col[min(e + edge_lanes * u, e1 - 1)];
-    float sum[kGradUnroll], before[kGradUnroll];
+    for (int u = 0; u < kEdgeUnroll; ++u) c[u] = col[min(e + edge_lanes * u, e1 - 1)];
+    float sum[kEdgeUnroll], before[kEdgeUnroll];
     if (add && q == 0) {
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u) before[u] = gw[min(e + edge_lanes * u, e1 - 1)];
+      for (int u = 0; u < kEdgeUnroll; ++u) before[u] = gw[min(e + edge_lanes * u, e1 - 1)];
     }
 #pragma unroll
-    for (int u = 0; u < kGradUnroll; ++u) sum[u] = 0.0f;
+    for (int u = 0; u < kEdgeUnroll; ++u) sum[u] = 0.0f;
     for (int64_t b0 = 0; b0 < B; b0 += kCols) {
       const int64_t b = b0 + q * VL;
       const bool have = b < B;
-      float g[VL], x[kGradUnroll][VL];
+      float g[VL], x[kEdgeUnroll][VL];
       load_row<VL>(gj + r * B + (have ? b : 0), g);
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u)
+      for (int u = 0; u < kEdgeUnroll; ++u)
         load_row<VL>(s.data + (have ? b : 0) * s.sb + c[u] * s.sn, x[u]);
 #pragma unroll
       for (int k = 0; k < VL; ++k) g[k] = have ? g[k] : 0.0f;
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u) {
+      for (int u = 0; u < kEdgeUnroll; ++u) {
 #pragma unroll
         for (int k = 0; k < VL; ++k)
           sum[u] = have ? __builtin_fmaf(g[k], x[u][k], sum[u]) : sum[u];
@@ -231,52 +208,12 @@ __global__ __launch_bounds__(kGradThreads) void weight_gradient_kernel(
 #pragma unroll
     for (int off = 1; off < LPE; off <<= 1) {
 #pragma unroll
-      for (int u = 0; u < kGradUnroll; ++u) sum[u] += __shfl_xor(sum[u], off, 64);
+      for (int u = 0; u < kEdgeUnroll; ++u) sum[u] += __shfl_xor(sum[u], off, 64);
     }
 #pragma unroll
-    for (int u = 0; u < kGradUnroll; ++u)
+    for (int u = 0; u < kEdgeUnroll; ++u)
       if (q == 0 && e + edge_lanes * u < e1)
         gw[e + edge_lanes * u] = add ? before[u] + sum[u] : sum[u];
-  }
-}
-
-// log2 of the edges a row's group takes at a time: the smallest power of two for
-// which kGradUnroll of them cover a row of average length, at most what fits
-// one wavefront beside the LPE lanes of an edge.
-inline int edge_lanes_for(int64_t edges, int64_t rows, int lpe) {
-  int lg = 0;
-  while ((lpe << lg) < 64 && (int64_t{kGradUnroll} << lg) * rows < edges) ++lg;
-  return lg;
-}
-
-struct EdgeForm {
-  int vl, lpe;
-};
-
-// The edge kernels' form for a batch: VL = 4 (2 at B = 2) where whole neuron-major
-// rows can be loaded, else one column per lane.
-inline EdgeForm edge_form(int64_t batch, bool whole_rows) {
-  if (whole_rows && batch == 2) return {2, 1};
-  if (whole_rows && batch % 4 == 0) return {4, batch == 4 ? 1 : batch == 8 ? 2 : 4};
-  return {1, batch <= 1 ? 1 : batch == 2 ? 2 : batch <= 4 ? 4 : batch <= 8 ? 8 : 16};
-}
-
-template <typename F>
-inline void with_edge_form(EdgeForm form, F&& launch) {
-  if (form.vl == 4) {
-    if (form.lpe == 1) launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
-    else if (form.lpe == 2) launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
-    else launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
-  } else if (form.vl == 2) {
-    launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
-  } else {
-    switch (form.lpe) {
-      case 1: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}); break;
-      case 2: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{}); break;
-      case 4: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{}); break;
-      case 8: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{}); break;
-      default: launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
-    }
   }
 }
 

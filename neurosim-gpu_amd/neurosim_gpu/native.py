@@ -37,7 +37,7 @@ import numpy as np
 import torch
 
 _LIB_NAME = "libneurosim_hip.so"
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 WEIGHT_F32, WEIGHT_F16, WEIGHT_E4M3, WEIGHT_NVFP4 = 0, 1, 2, 3
 _PLAN_CACHE = 64   # row plans kept per extension (one per live topology and batch width)
@@ -114,9 +114,10 @@ class _EventArgs(ctypes.Structure):
                 ("out_adaptation", _OutPlane), ("out_emitted", _OutPlane),
                 ("delta", _c_ptr), ("pending_in", _c_ptr), ("pending_out", _c_ptr),
                 ("out_weight", _c_ptr), ("flags", ctypes.c_int32), ("reserved", ctypes.c_int32),
-                ("activity", _c_ptr)]
+                ("activity", _c_ptr), ("in_rowptr", _c_ptr), ("in_col", _c_ptr),
+                ("emitting", _c_ptr)]
 
-EVENT_ADVANCE_ONLY = 1   # NS_EVENT_ADVANCE_ONLY
+EVENT_ADVANCE_ONLY, EVENT_PRODUCT = 1, 4   # NS_EVENT_*
 EVENT_ACTIVITY_SLOTS = 32   # NS_EVENT_ACTIVITY_SLOTS
 EVENT_ACTIVITY_STRIDE = 16  # NS_EVENT_ACTIVITY_STRIDE
 
@@ -1430,10 +1431,13 @@ class PreparedEvent:
     planes and writes the per-tick words: planes, the pending buffers of
     ``parity`` (0 or 1; None without pending buffers), the source-major weight
     copy, the advance-only flag and the activity counters of a sampled tick.
-    The results equal ``NativeExtension.dendritic_event`` on the same inputs."""
+    ``in_view`` (in_rowptr, in_col and a bitmap workspace) allows ``product``: an
+    advance-only tick followed, in the same call, by current += W @ delta
+    (NS_EVENT_PRODUCT).  The results equal ``NativeExtension.dendritic_event`` on the same inputs."""
 
     def __init__(self, extension: "NativeExtension", state: torch.Tensor, params, theta, rowptr,
-                 dst, weight_index, weight, delta=None, pending=None, activity=None):
+                 dst, weight_index, weight, delta=None, pending=None, activity=None,
+                 in_view=None):
         _check_state(state)
         self.lib = extension.lib
         args = _EventArgs()
@@ -1468,11 +1472,25 @@ class PreparedEvent:
                 or activity.device != state.device):
             raise RuntimeError("activity must hold EVENT_ACTIVITY_SLOTS * "
                                "EVENT_ACTIVITY_STRIDE int64 counters on the state's device")
+        self._in_view = in_view
+        if in_view is not None:
+            in_rowptr, in_col, emitting = in_view
+            for index in (in_rowptr, in_col):
+                _index(index, state)
+            if (in_rowptr.numel() != n + 1 or in_col.numel() != weight.numel()
+                    or emitting.dtype != torch.int64 or not emitting.is_contiguous()
+                    or emitting.numel() < (batch * n + 63) // 64
+                    or emitting.device != state.device):
+                raise RuntimeError("invalid destination-major view of the event topology")
+            args.in_rowptr, args.in_col = in_rowptr.data_ptr(), in_col.data_ptr()
+            args.emitting = emitting.data_ptr()
         self.args, self._ref = args, ctypes.byref(args)
         self.batch, self.n, self.shape, self.device = batch, n, state.shape, state.device
         self.params = tuple(params)
-        self._fixed = (theta, rowptr, dst, weight_index, weight, pending, activity, *self.params)
-        self._addressed = (*self.params, theta, rowptr, dst, weight_index, weight)
+        self._fixed = (theta, rowptr, dst, weight_index, weight, pending, activity, in_view,
+                       *self.params)
+        self._addressed = (*self.params, theta, rowptr, dst, weight_index, weight,
+                           *(in_view or ()))
         self._pointers = tuple(map(_data_ptr, self._addressed))
         self._delta = delta
         self._pending = ((pending[0].data_ptr(), pending[1].data_ptr())
@@ -1483,9 +1501,9 @@ class PreparedEvent:
         self._last = None     # (s', d', a', e', their words)
 
     def matches(self, state, params, theta, rowptr, dst, weight_index, weight, pending=None,
-                activity=None) -> bool:
-        given = (theta, rowptr, dst, weight_index, weight, pending, activity, *params)
-        if len(given) != 13 or not all(map(is_, given, self._fixed)):
+                activity=None, in_view=None) -> bool:
+        given = (theta, rowptr, dst, weight_index, weight, pending, activity, in_view, *params)
+        if len(given) != 14 or not all(map(is_, given, self._fixed)):
             return False
         last = self._last
         if (last is None or state is not last[0]) and state.shape != self.shape:
@@ -1494,7 +1512,7 @@ class PreparedEvent:
 
     def __call__(self, state, dendrite, adaptation, emitted, current, drive, drive_scalar,
                  dendritic_drive, dendritic_scalar, *, parity=None, advance_only=False,
-                 sample=False, out_weight=None) -> tuple:
+                 sample=False, out_weight=None, product=False) -> tuple:
         """One tick; drives are validated [B,N] views or None with a scalar."""
         last = self._last
         if (last is not None and state is last[0] and dendrite is last[1]
@@ -1539,6 +1557,9 @@ class PreparedEvent:
             pending_in, pending_out = self._pending[parity], self._pending[1 - parity]
             if advance_only:
                 pending_out = 0
+        if product and (self._in_view is None or not advance_only or parity is None):
+            raise RuntimeError("the product needs the destination-major view and a fused "
+                               "advance-only tick")
         if sample and not self._activity:
             raise RuntimeError("this tick was prepared without activity counters")
         delta = 0
@@ -1548,7 +1569,9 @@ class PreparedEvent:
                                           device=self.device)
             delta = self._delta.data_ptr()
         _EVENT_TAIL.pack_into(args, _EVENT_TAIL_AT, delta, pending_in, pending_out,
-                              self._out_weight[1], EVENT_ADVANCE_ONLY if advance_only else 0,
+                              self._out_weight[1],
+                              (EVENT_ADVANCE_ONLY if advance_only else 0)
+                              | (EVENT_PRODUCT if product else 0),
                               0, self._activity if sample else 0)
         batch, n = self.batch, self.n
         outs, base = _new_outputs(4, batch, n, self.device)

@@ -696,6 +696,26 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
         return self.state
 
 
+# Fewest edges times columns for which the scatter's tick may become an advance and
+# an in-edge product (NS_EVENT_PRODUCT).  Below, an eager tick is bound by its host
+# side, which a second launch makes longer (N=50k, M=1M, B=1: 12.7 us per scattered
+# tick at 12% activity, 19.6 with the product).
+PRODUCT_MIN_EDGES = 4_000_000
+
+
+def product_break_even(n_edges: int, batch: int) -> float:
+    """Active out-edges of a tick from which the in-edge product beats the scatter.
+
+    The scatter's cost is its atomics, the product's the stream of the edges.
+    Crossings measured (N, M, B, thousands of active out-edges): 50k 4M 1, 180;
+    166k 10M 1, 380; 300k 15M 1, 610; 166k 25M 1, 960; 50k 2M 3, 310; 100k 4M 5,
+    1030; and where the scatter adds runs of columns, 60k 5M 2, 180; 60k 3M 4,
+    370; 50k 1M 8, 260; 60k 3M 16, 1070.  At 12% activity, us per tick, scatter /
+    product: 166k 10M 1, 68 / 29; 166k 25M 1, 164 / 62; 50k 1M 8, 41 / 19."""
+    runs = 2 <= batch <= 64 and batch & (batch - 1) == 0
+    return 100_000 + (0.02 if runs else 0.034) * n_edges * batch
+
+
 class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
     """The PELS event tick on the device, by default in one HIP launch.
 
@@ -707,7 +727,12 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
     the current as it reads it (j = current + pending, the same float32 sum
     either way).  Reading ``persistent_current`` folds the outstanding buffer
     first, so the attribute always holds W @ emitted as in the reference;
-    assigning it discards the outstanding buffer.  The scatter streams a
+    assigning it discards the outstanding buffer.  On a graph of at least
+    ``PRODUCT_MIN_EDGES`` edges times columns an eager tick counts its active
+    out-edges every ``policy_interval`` ticks (on the device, read back without
+    waiting), and while they exceed ``product_break_even`` the deltas propagate by
+    a second launch that sums each destination's in-edges from the emitting
+    sources, without atomics: the same sums in another order.  The scatter streams a
     source-major copy of the weights (M floats, rebuilt when the weights
     change; ``source_major_weights.enabled = False`` gathers through
     ``out_weight_index`` instead).  Ticks captured in a HIP
@@ -778,11 +803,22 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
             self._delta = torch.empty(batch * n, dtype=torch.float32, device=device)
         # The path the next tick takes; "auto" changes it from sampled activity.
         self._path = "matrix" if propagation == "matrix" else "event"
+        # The scatter's ticks move to the in-edge product while many pairs emit.
+        self._adaptive = (propagation == "event" and self._pending is not None and batch > 0
+                          and topology.n_edges * batch >= PRODUCT_MIN_EDGES)
+        self._gather = False
+        self._in_view = None
+        if self._adaptive:
+            self._delta = torch.empty(batch * n, dtype=torch.float32, device=device)
         self._activity = self._activity_host = self._sample = None
-        if propagation == "auto":
+        if propagation == "auto" or self._adaptive:
             slots = EVENT_ACTIVITY_SLOTS * EVENT_ACTIVITY_STRIDE
             self._activity = torch.zeros(slots, dtype=torch.int64, device=device)
             self._activity_host = torch.zeros(slots, dtype=torch.int64, pin_memory=True)
+            self._activity_counts = self._activity_host.numpy().reshape(EVENT_ACTIVITY_SLOTS,
+                                                                        EVENT_ACTIVITY_STRIDE)
+            self._activity_seen = 0
+            self._sampled = torch.cuda.Event()
         # The matrix propagation's product kernel and, for panels, its layout.
         if kernel == "panels" and (batch not in (1, 2) or not native):
             raise ValueError("the panel kernel needs batch 1 or 2 and the native extension")
@@ -823,21 +859,44 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
         return self._product_struct
 
     def _policy_tick(self) -> bool:
-        """For "auto": apply a finished sample at a policy tick and say whether
-        this tick samples (counts its active out-edges)."""
-        if self.propagation != "auto" or self._tick % self.policy_interval:
-            return False
+        """Apply a finished sample and say whether this tick samples (counts its
+        active out-edges).  "auto" does so at policy ticks; the scatter of a large
+        graph (``_adaptive``) applies a sample on the first tick that finds it done."""
+        phase = self._tick % self.policy_interval
+        if self._adaptive:
+            due = phase == self.policy_interval // 2     # past the start state's transient
+            if not due and self._sample is None:
+                return False
+        else:
+            due = phase == 0
+            if self.propagation != "auto" or not due:
+                return False
         if torch.cuda.is_current_stream_capturing():
             return False
         if self._sample is not None:
             if not self._sample.query():
                 return False                 # the last sample is still on its way
-            counts = self._activity_host.view(EVENT_ACTIVITY_SLOTS, EVENT_ACTIVITY_STRIDE)
-            edges = int(counts[:, 0].sum())
-            slots = max(self.topology.n_edges * self.state.shape[0], 1)
-            self._path = "event" if edges / slots < self.event_edge_fraction else "matrix"
+            # The counters only grow: a sample is what they grew by.
+            total = int(self._activity_counts[:, 0].sum())
+            edges, self._activity_seen = total - self._activity_seen, total
+            if self._adaptive:
+                self._gather = edges >= product_break_even(self.topology.n_edges,
+                                                           self.state.shape[0])
+            else:
+                slots = max(self.topology.n_edges * self.state.shape[0], 1)
+                self._path = "event" if edges / slots < self.event_edge_fraction else "matrix"
             self._sample = None
-        return True
+        return due
+
+    def _destinations(self) -> tuple:
+        """The destination-major view for the in-edge product and its bitmap."""
+        topology = self.topology
+        view = self._in_view
+        if view is None or view[0] is not topology.in_rowptr or view[1] is not topology.in_col:
+            words = torch.empty((self._delta.numel() + 63) // 64, dtype=torch.int64,
+                                device=self._delta.device)
+            view = self._in_view = (topology.in_rowptr, topology.in_col, words)
+        return view
 
     @property
     def persistent_current(self) -> torch.Tensor:
@@ -904,7 +963,9 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
         native = isinstance(self.extension, NativeExtension)
         sample = self._policy_tick()
         matrix = native and self._path == "matrix"
-        out_weight = self._source_major() if not matrix else None
+        # Inside a capture the scatter stays: no replay could follow the activity.
+        gather = self._gather and not torch.cuda.is_current_stream_capturing()
+        out_weight = self._source_major() if not (matrix or gather) else None
         topology, params = self.topology, self._parameters()
         if native:
             # One launch with pending buffers: pending[parity] holds the last tick's
@@ -913,15 +974,18 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
             tick = self._prepared
             fixed = (self.theta, topology.out_rowptr, topology.dst, topology.out_weight_index,
                      topology.in_weight)
+            in_view = self._destinations() if self._adaptive else None
             if tick is None or not tick.matches(self.state, params, *fixed,
-                                                pending=self._pending, activity=self._activity):
+                                                pending=self._pending, activity=self._activity,
+                                                in_view=in_view):
                 tick = self._prepared = PreparedEvent(self.extension, self.state, params, *fixed,
                                                       delta=self._delta, pending=self._pending,
-                                                      activity=self._activity)
+                                                      activity=self._activity, in_view=in_view)
             outs = tick(self.state, self.dendritic_state, self.adaptation_state,
                         self.emitted_state, self._current, u, us, v, vs,
                         parity=self._parity if self._pending is not None else None,
-                        advance_only=matrix, sample=sample, out_weight=out_weight)
+                        advance_only=matrix or gather, sample=sample, out_weight=out_weight,
+                        product=gather)
         else:
             extra = {"out_weight": out_weight} if out_weight is not None else {}
             outs = self.extension.dendritic_event(
@@ -945,12 +1009,11 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
                     topology.in_weight, self._current, panels)
             product()
         if sample:
-            # The counters reach the host behind this tick; a later policy tick
-            # reads them once the copy is done, then they start again from zero.
+            # The counters reach the host behind this tick; a later tick reads them
+            # once the copy is done.
             self._activity_host.copy_(self._activity, non_blocking=True)
-            self._sample = torch.cuda.Event()
+            self._sample = self._sampled
             self._sample.record()
-            self._activity.zero_()
         if self._pending is not None:
             self._parity ^= 1
         self._tick += 1

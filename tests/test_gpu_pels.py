@@ -382,3 +382,122 @@ def test_csr_spmm_accumulates_in_place(gpu, batch):
     with pytest.raises(RuntimeError, match="must not overlap itself"):
         native.extension.csr_spmm(source, t.in_rowptr, t.in_col, t.in_weight,
                                   accumulate_into=torch.zeros(1, device=gpu).expand(batch, 2000))
+
+
+@pytest.fixture
+def always_gather(monkeypatch):
+    """Every large-graph rule set so that a sampled tick turns to the in-edge product."""
+    from neurosim_gpu import native_compartmental as nc
+
+    monkeypatch.setattr(nc, "PRODUCT_MIN_EDGES", 0)
+    monkeypatch.setattr(nc, "product_break_even", lambda n_edges, batch: 1.0)
+
+
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 5, 8, 12, 16, 17])
+@pytest.mark.parametrize("theta", [0.0, 0.01])
+def test_in_edge_product_matches_the_scatter(gpu, always_gather, batch, theta):
+    """The event tick's in-edge product (NS_EVENT_PRODUCT: the emitting pairs' bitmap at
+    batch 1 and 2, whole or single columns per lane from 3 on) on an odd number of
+    neurons with hub destinations and empty rows, against the oracle and the exact
+    current; ticks before the first sample scatter, and reads and assignments of the
+    current fall between the two."""
+    from oracle import topology as otop
+    from neurosim_gpu import SparseTopology, topology_to
+    from cases import model_to, standard_model
+
+    print(f"case pels in-edge product B={batch} theta={theta}", flush=True)
+    n = 1301
+    rng = np.random.default_rng(5)
+    src, dst = [rng.integers(0, n, 9 * n)], [rng.integers(0, n - 40, 9 * n)]
+    for target, degree in ((3, 1200), (64, 700), (n - 1, 300)):
+        src.append(rng.permutation(n)[:degree])
+        dst.append(np.full(degree, target))
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    weight = (rng.standard_normal(src.size) * 0.02).astype(np.float32)
+    graph = otop.build(n, src, dst, weight)
+    topology = topology_to(SparseTopology.from_edges(n, torch.from_numpy(src), torch.from_numpy(dst),
+                                                     torch.from_numpy(weight)), gpu)
+    model, params = standard_model(n)
+    columns = torch.linspace(0.0, 1.0, batch)[:, None]
+    state = 0.1 + 0.05 * columns.expand(batch, n).contiguous()
+    native = NativeDendriticPELSRuntime(topology, model_to(model, gpu), state.to(gpu), theta=theta,
+                                        policy_interval=4)
+    oracle = ort.PelsOracle(graph, params, state, theta=theta)
+    matrix = ort.csr_matrix(graph)
+    per_neuron = torch.from_numpy(rng.uniform(0.0, 0.2, n).astype(np.float32))
+    gathered = 0
+    for tick in range(30):
+        drive = (0.3 if tick < 20 else 0.05) * (0.5 + columns) + per_neuron
+        native.step(drive.to(gpu), dendritic_drive=0.1)
+        oracle.step(drive, 0.1)
+        gathered += native._gather
+        torch.cuda.synchronize()
+        if tick % 9 == 4:
+            exact = ort.propagate(matrix, native.emitted_state.cpu())
+            assert max_err(native.persistent_current, exact) <= 1e-5
+        if tick == 15:
+            native.persistent_current = ort.propagate(matrix, native.emitted_state.cpu()).to(gpu)
+    assert gathered >= 20 and native.last_backend == "native" and native.selected_path == "event"
+    assert state_error(native, oracle) <= (1e-5 if theta == 0 else 1e-3)
+    exact = ort.propagate(matrix, native.emitted_state.cpu())
+    assert max_err(native.persistent_current, exact) <= 1e-5
+
+
+def test_in_edge_product_follows_activity_weights_and_captures(gpu, always_gather):
+    """The product is left again when activity falls; an in-place weight edit and a new
+    weight version are followed at once; a capture takes the scatter; and a silent
+    source's infinite weight pushes nothing, as in the scatter."""
+    print("case pels in-edge product switches", flush=True)
+    case = make_case(3000, 60_000, 8, gpu)
+    topology = case.topology
+    topology.in_weight[5] = float("inf")
+    silent = int(topology.in_col[5])
+    start = torch.full((1, 3000), 0.1, device=gpu)
+    theta = torch.full((3000,), 0.005, device=gpu)
+    theta[silent] = 100.0
+    # the source's other uses: a finite current to start from
+    native = NativeDendriticPELSRuntime(topology, case.model, start, theta=theta,
+                                        policy_interval=2)
+    two = NativeDendriticPELSRuntime(topology, case.model, start, theta=theta, one_launch=False)
+    for runtime in (native, two):
+        runtime.persistent_current = torch.zeros(1, 3000, device=gpu)
+    fields = ("state", "dendritic_state", "adaptation_state", "emitted_state")
+
+    def same():
+        for f in fields:
+            assert max_err(getattr(native, f), getattr(two, f)) <= 2e-2 and \
+                float((getattr(native, f) - getattr(two, f)).abs().mean()) <= 1e-5, f
+        assert bool(torch.isfinite(native.persistent_current).all())
+        assert float((native.persistent_current - two.persistent_current).abs().mean()) <= 1e-5
+
+    for tick in range(24):
+        if tick == 8:
+            with torch.no_grad():
+                topology.in_weight.mul_(0.5)
+        for runtime in (native, two):
+            runtime.step(0.3 if tick % 2 else 0.1, dendritic_drive=0.1)
+        torch.cuda.synchronize()
+        same()
+    assert native._gather
+    replayed = [getattr(native, f) for f in fields]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(4):
+            native.step(0.2, dendritic_drive=0.1)
+    end = [getattr(native, f) for f in fields]
+    for replay in range(3):
+        graph.replay()
+        for _ in range(4):
+            two.step(0.2, dendritic_drive=0.1)
+        torch.cuda.synchronize()
+        same()
+        for a, b in zip(replayed, end):
+            a.copy_(b)
+    from neurosim_gpu import native_compartmental as nc
+    nc.product_break_even = lambda n_edges, batch: 1e12
+    for _ in range(6):
+        for runtime in (native, two):
+            runtime.step(0.2, dendritic_drive=0.1)
+        torch.cuda.synchronize()
+    assert not native._gather
+    same()
