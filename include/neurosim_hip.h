@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define NS_ABI_VERSION 21
+#define NS_ABI_VERSION 22
 
 /* Return codes. */
 #define NS_OK 0
@@ -239,7 +239,39 @@ typedef struct ns_step_args {
   ns_out_plane out_adaptation; /* a_{t+1} */
   ns_out_plane out_current;    /* optional: j = W @ s_t as well (data NULL: not written);
                                   a recorded tick keeps it for its backward */
+  const struct ns_rollout* rollout;  /* optional: many ticks in one launch (NULL: one) */
 } ns_step_args;
+
+/* Many ticks of a small network in one launch (ns_step_args.rollout; `plan` and
+ * `panels` are then not read): one workgroup per column holds that column's
+ * edges in registers and its states in registers and LDS for the whole run.  The
+ * states are the planes of the args, before the first and after the last tick;
+ * an output plane may be its input plane (same data and strides).
+ *
+ * Rows are summed as the row-block tick sums them: a row has `slices` (a power of
+ * two, at most 64) tasks; task h takes the row's edges h, h + slices, ...  Tasks
+ * lie in chunks of 64, one wavefront's lanes, all of one `slices`, a row's tasks
+ * on neighbouring lanes from a multiple of `slices` on.  Each of the 16
+ * wavefronts walks its chunks (`n_rounds` of them, the last ones possibly empty). */
+typedef struct ns_rollout {
+  int32_t ticks;               /* > 0 */
+  int32_t slots;               /* edges per lane held in registers: 16, 32 or 48 */
+  int32_t n_rounds;            /* chunks per wavefront */
+  int32_t reserved;
+  const int32_t* tasks;        /* [16][n_rounds][64] pairs: first CSR edge; edge count in the
+                                  low 16 bits and row in the high 16 (0xFFFF: no task) */
+  const int32_t* rounds;       /* [16][n_rounds]: quads of edges per lane (0: no chunk) in the
+                                  low 16 bits, log2 slices in the high 16; at most slots / 4
+                                  quads per wavefront */
+  int64_t drive_tick;          /* floats from one tick's drive plane to the next (0: the same */
+  int64_t dendritic_tick;      /* plane every tick) */
+  ns_out_plane trace;          /* optional: s after each tick, [B,N] at trace.data + */
+  int64_t trace_tick;          /* t * trace_tick floats (data NULL: not written) */
+} ns_rollout;
+
+/* Largest network of a rollout launch. */
+#define NS_ROLLOUT_MAX_NEURONS 2048
+#define NS_ROLLOUT_MAX_ROUNDS 7
 
 /* Arguments of one PELS event tick (advance + emit, then scatter). */
 typedef struct ns_event_args {

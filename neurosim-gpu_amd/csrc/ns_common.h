@@ -118,4 +118,22 @@ __device__ __forceinline__ float nvfp4_weight(uint32_t nibble, float block_times
   return e2m1_pair(nibble & 15u).x * block_times_global;
 }
 
+// Weight of CSR edge e, decoded (gscale: the decoded global scale of E4M3 and
+// NVFP4 weights).
+template <int FMT>
+__device__ __forceinline__ float csr_weight(const void* weight, const uint8_t* scales, int64_t e,
+                                            float gscale) {
+  if constexpr (FMT == NS_WEIGHT_F32) {
+    return static_cast<const float*>(weight)[e];
+  } else if constexpr (FMT == NS_WEIGHT_F16) {
+    return static_cast<float>(static_cast<const _Float16*>(weight)[e]);
+  } else if constexpr (FMT == NS_WEIGHT_E4M3) {
+    return e4m3_to_float(static_cast<const uint8_t*>(weight)[e]) * gscale;
+  } else {
+    const uint32_t byte = static_cast<const uint8_t*>(weight)[e >> 1];
+    const float bs = e4m3_to_float(scales[e >> 4]) * gscale;
+    return nvfp4_weight((byte >> (4 * (e & 1))) & 15u, bs);
+  }
+}
+
 }  // namespace ns

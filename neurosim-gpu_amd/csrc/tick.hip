@@ -109,33 +109,8 @@ __device__ __forceinline__ void load_quad(const TickArgs& A, int64_t q, bool vec
     w[k] = 0.0f;
     if (e < A.M) {
       c[k] = A.col[e];
-      if constexpr (FMT == NS_WEIGHT_F32) {
-        w[k] = static_cast<const float*>(A.weight)[e];
-      } else if constexpr (FMT == NS_WEIGHT_F16) {
-        w[k] = static_cast<float>(static_cast<const _Float16*>(A.weight)[e]);
-      } else if constexpr (FMT == NS_WEIGHT_E4M3) {
-        w[k] = e4m3_to_float(static_cast<const uint8_t*>(A.weight)[e]) * gscale;
-      } else {
-        const uint32_t byte = static_cast<const uint8_t*>(A.weight)[e >> 1];
-        const float bs = e4m3_to_float(A.scales[e >> 4]) * gscale;
-        w[k] = nvfp4_weight((byte >> (4 * (e & 1))) & 15u, bs);
-      }
+      w[k] = csr_weight<FMT>(A.weight, A.scales, e, gscale);
     }
-  }
-}
-
-template <int FMT>
-__device__ __forceinline__ float load_weight(const TickArgs& A, int64_t e, float gscale) {
-  if constexpr (FMT == NS_WEIGHT_F32) {
-    return static_cast<const float*>(A.weight)[e];
-  } else if constexpr (FMT == NS_WEIGHT_F16) {
-    return static_cast<float>(static_cast<const _Float16*>(A.weight)[e]);
-  } else if constexpr (FMT == NS_WEIGHT_E4M3) {
-    return e4m3_to_float(static_cast<const uint8_t*>(A.weight)[e]) * gscale;
-  } else {
-    const uint32_t byte = static_cast<const uint8_t*>(A.weight)[e >> 1];
-    const float bs = e4m3_to_float(A.scales[e >> 4]) * gscale;
-    return nvfp4_weight((byte >> (4 * (e & 1))) & 15u, bs);
   }
 }
 
@@ -166,7 +141,7 @@ __device__ void rows_one_by_one(const TickArgs& A, int r0, int r1, int b0, float
 #pragma unroll
     for (int j = 0; j < BT; ++j) acc[j] = 0.0f;
     for (int64_t e = rs + tid; e < re; e += kThreads) {
-      const float w = load_weight<FMT>(A, e, gscale);
+      const float w = csr_weight<FMT>(A.weight, A.scales, e, gscale);
       const int64_t c = A.col[e];
 #pragma unroll
       for (int j = 0; j < BT; ++j)
@@ -433,6 +408,7 @@ hipError_t launch_tick(const TickArgs& A, int fmt, hipStream_t stream) {
 }
 
 int panel_step(const ns_step_args& a, hipStream_t stream, int product, bool launch);
+int rollout_step(const ns_step_args& a, hipStream_t stream);
 
 // Host-side validation shared by the tick and the plain product.
 int check_csr(const ns_csr& m, int64_t n) {
@@ -543,6 +519,7 @@ extern "C" int ns_dendritic_step(const ns_step_args* args, void* stream) {
   if (!args) return fail("arguments are required");
   const ns_step_args& a = *args;
   if (int rc = check_step_head(a)) return rc;
+  if (a.rollout) return rollout_step(a, static_cast<hipStream_t>(stream));
   if (!a.panels)
     if (int rc = check_matrix(a.matrix, a.n_neurons, a.plan, a.batch)) return rc;
   if (a.batch == 0) return NS_OK;  // empty planes may carry null pointers

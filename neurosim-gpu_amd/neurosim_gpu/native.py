@@ -37,7 +37,7 @@ import numpy as np
 import torch
 
 _LIB_NAME = "libneurosim_hip.so"
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 WEIGHT_F32, WEIGHT_F16, WEIGHT_E4M3, WEIGHT_NVFP4 = 0, 1, 2, 3
 _PLAN_CACHE = 64   # row plans kept per extension (one per live topology and batch width)
@@ -98,7 +98,19 @@ class _StepArgs(ctypes.Structure):
                 ("params", _Vector * 6), ("matrix", _Csr), ("plan", _RowPlan),
                 ("panels", _c_ptr),
                 ("out_state", _OutPlane), ("out_dendrite", _OutPlane),
-                ("out_adaptation", _OutPlane), ("out_current", _OutPlane)]
+                ("out_adaptation", _OutPlane), ("out_current", _OutPlane),
+                ("rollout", _c_ptr)]
+
+
+class _Rollout(ctypes.Structure):
+    _fields_ = [("ticks", ctypes.c_int32), ("slots", ctypes.c_int32),
+                ("n_rounds", ctypes.c_int32), ("reserved", ctypes.c_int32),
+                ("tasks", _c_ptr), ("rounds", _c_ptr), ("drive_tick", _c_i64),
+                ("dendritic_tick", _c_i64), ("trace", _OutPlane), ("trace_tick", _c_i64)]
+
+ROLLOUT_MAX_NEURONS, ROLLOUT_MAX_ROUNDS = 2048, 7   # NS_ROLLOUT_*
+ROLLOUT_SLOTS = (16, 32, 48)
+ROLLOUT_WAVES = 16
 
 
 class _EventArgs(ctypes.Structure):
@@ -1104,6 +1116,121 @@ class TickLauncher:
                                                        stream), self.lib)
         else:
             _raise_on(self.lib.ns_dendritic_step(ctypes.byref(args), stream), self.lib)
+
+
+def plan_rollout(rowptr: np.ndarray, bounds: np.ndarray, batch: int):
+    """Tasks of a one-launch rollout (ns_rollout) for a graph and its row plan.
+
+    ``rowptr`` [N+1] and ``bounds`` [blocks+1, 2] are host arrays.  Returns (slots,
+    tasks int32 [16, rounds, 64, 2], rounds int32 [16, rounds]), or None when the
+    network does not fit: too many neurons, a row block that the row kernel reduces
+    row by row, or more edges than the lanes' registers hold.
+
+    A row has the slices the row-block kernel gives it, a function of its block's
+    row count and the column tile; rows are sorted by slices and length, so that a
+    chunk of 64 tasks is of one kind and of similar length, and the chunks go to the
+    wavefronts longest first, each to the one with the fewest quads."""
+    n = rowptr.size - 1
+    if not 0 < n <= ROLLOUT_MAX_NEURONS:
+        return None
+    tile = 1 if batch <= 1 else 2 if batch <= 2 else 4 if batch <= 4 else 8 if batch <= 8 else 16
+    capacity = int(load_library().ns_block_edges(int(batch)))
+    first_row, first_edge = bounds[:, 0].astype(np.int64), bounds[:, 1].astype(np.int64)
+    counts = np.diff(first_row)
+    edges = first_edge[1:] - (first_edge[:-1] & ~3)
+    if counts.size == 0 or np.any(counts > 256) or np.any(edges > capacity):
+        return None
+    slices = np.ones(n, np.int64)
+    for block, rows in enumerate(counts):
+        if rows:
+            group = min(64, 1 << ((256 // int(rows)).bit_length() - 1))
+            slices[first_row[block]:first_row[block + 1]] = max(1, group // tile)
+    start = rowptr[:-1].astype(np.int64)
+    degree = rowptr[1:].astype(np.int64) - start
+    chunks = []                                    # (quads, log2 slices, tasks [64, 2])
+    for width in np.unique(slices):
+        rows = np.flatnonzero(slices == width)
+        rows = rows[np.argsort(-degree[rows], kind="stable")]
+        part = np.arange(width)
+        count = np.maximum(0, (degree[rows][:, None] - part + width - 1) // width)
+        tasks = np.stack((start[rows][:, None] + part,
+                          count | (rows[:, None] << 16)), axis=-1).reshape(-1, 2)
+        pad = -tasks.shape[0] % 64
+        tasks = np.concatenate((tasks, np.tile(np.array([[0, 0xFFFF << 16]]), (pad, 1))))
+        lengths = np.concatenate((count.reshape(-1), np.zeros(pad, np.int64)))
+        for k in range(0, tasks.shape[0], 64):
+            quads = max(1, int(-(-lengths[k:k + 64].max() // 4)))
+            chunks.append((quads, int(width).bit_length() - 1, tasks[k:k + 64]))
+    chunks.sort(key=lambda c: -c[0])
+    load, mine = [0] * ROLLOUT_WAVES, [[] for _ in range(ROLLOUT_WAVES)]
+    for chunk in chunks:
+        wave = load.index(min(load))
+        load[wave] += chunk[0]
+        mine[wave].append(chunk)
+    slots = next((s for s in ROLLOUT_SLOTS if 4 * max(load) <= s), None)
+    n_rounds = max(map(len, mine))
+    if slots is None or n_rounds > ROLLOUT_MAX_ROUNDS:
+        return None
+    tasks = np.zeros((ROLLOUT_WAVES, n_rounds, 64, 2), np.int64)
+    tasks[..., 1] = 0xFFFF << 16
+    rounds = np.zeros((ROLLOUT_WAVES, n_rounds), np.int32)
+    for wave, own in enumerate(mine):
+        for r, (quads, log2, chunk) in enumerate(own):
+            tasks[wave, r] = chunk
+            rounds[wave, r] = quads | (log2 << 16)
+    return slots, tasks.astype(np.uint32).view(np.int32), rounds
+
+
+class RolloutLauncher:
+    """``ticks`` ticks of a ``TickLauncher`` on row blocks in one launch (ns_rollout).
+
+    ``build`` gives None where the network does not fit a compute unit per column
+    (``plan_rollout``), the batch exceeds the compute units, or the launcher runs on
+    panels or bands.  The states are updated in place in ``planes``; the drives and
+    the trace are fixed at construction."""
+
+    def __init__(self, launcher: TickLauncher, plan: tuple, ticks: int, planes: tuple,
+                 staged: tuple, trace: torch.Tensor | None) -> None:
+        slots, tasks, rounds = plan
+        device = planes[0].device
+        self.lib, self.device = launcher.lib, device
+        args = _StepArgs.from_buffer_copy(launcher.args)
+        rollout = _Rollout(ticks, slots, rounds.shape[1], 0)
+        self._tables = (_device_tensor(tasks, device), _device_tensor(rounds, device))
+        rollout.tasks, rollout.rounds = (t.data_ptr() for t in self._tables)
+        for name, view, fixed in (("drive", staged[0], launcher.fixed_drives[0]),
+                                  ("dendritic_drive", staged[1], launcher.fixed_drives[1])):
+            tick = 0
+            if view is not None:
+                fixed, tick = _plane(view[0], planes[0], "drive"), view.stride(0)
+            setattr(args, name, fixed)
+            setattr(rollout, "drive_tick" if name == "drive" else "dendritic_tick", tick)
+        if trace is not None:
+            rollout.trace = _out(trace[0])
+            rollout.trace_tick = trace.stride(0)
+        for name, value in zip(("state", "dendrite", "adaptation"), planes):
+            setattr(args, name, _plane(value, planes[0], name))
+            setattr(args, "out_" + name, _out(value))
+        args.rollout = ctypes.addressof(rollout)
+        self.args, self._ref = args, ctypes.byref(args)
+        self._keep = (launcher, rollout, planes, staged, trace)
+
+    @classmethod
+    def build(cls, extension: "NativeExtension", launcher: TickLauncher, rowptr: torch.Tensor,
+              ticks: int, planes: tuple, staged: tuple, trace) -> "RolloutLauncher | None":
+        batch, n = launcher.batch, launcher.n
+        if launcher.bands is not None or launcher.args.panels or n > ROLLOUT_MAX_NEURONS:
+            return None
+        device = planes[0].device
+        if batch > torch.cuda.get_device_properties(device).multi_processor_count:
+            return None
+        bounds, blocks, _ = extension.plan_tensors(rowptr, batch)
+        plan = plan_rollout(rowptr.detach().to("cpu", torch.int32).numpy(),
+                            bounds.cpu().numpy().reshape(blocks + 1, 2), batch)
+        return cls(launcher, plan, ticks, planes, staged, trace) if plan is not None else None
+
+    def __call__(self) -> None:
+        _raise_on(self.lib.ns_dendritic_step(self._ref, current_stream(self.device)), self.lib)
 
 
 def current_stream(device: torch.device) -> int:

@@ -3,7 +3,9 @@
 A rollout owns two sets of neuron-major state planes and alternates between
 them: tick i reads set i % 2 and writes set (i+1) % 2, so an even number of
 ticks ends where it started and the captured graph can be replayed back to
-back with no copy, no allocation and no host work per tick.
+back with no copy, no allocation and no host work per tick.  A network small
+enough for one compute unit per column runs the whole chunk in one launch instead
+(``RolloutLauncher``), in place on the first set.
 
 Inputs can be staged per tick, as in the reference's CUDA-graph rollout of its
 drift benchmark (benchmarks/precision_drift.py:74-143): a drive given as a
@@ -17,7 +19,7 @@ from __future__ import annotations
 
 import torch
 
-from .native import NativeExtension, TickLauncher, drive_plane, new_planes
+from .native import NativeExtension, RolloutLauncher, TickLauncher, drive_plane, new_planes
 
 
 def _per_tick(value, ticks: int, batch: int, n: int, state: torch.Tensor, what: str):
@@ -89,7 +91,12 @@ class MatrixRollout:
                       if trace else None)
         self.reset_from_runtime()
         self.graph = None
-        if use_graph:
+        # A network that fits a compute unit per column runs all its ticks in one
+        # launch, bitwise the row-block ticks.
+        self._resident = (RolloutLauncher.build(extension, self._launch, topology.in_rowptr, ticks,
+                                                self._sets[0], staged, self.trace)
+                          if use_graph else None)
+        if use_graph and self._resident is None:
             self._capture()
 
     def _eager(self, count: int | None = None) -> None:
@@ -134,7 +141,9 @@ class MatrixRollout:
     def run(self, repeats: int = 1) -> None:
         """Advance ``repeats * ticks`` ticks (asynchronous on the current stream)."""
         for _ in range(repeats):
-            if self.graph is not None:
+            if self._resident is not None:
+                self._resident()
+            elif self.graph is not None:
                 self.graph.replay()
             else:
                 self._eager()

@@ -598,3 +598,81 @@ def test_row_block_size_follows_the_graph():
         for m in (0, 1, 10**3, 10**5, 10**7):
             edges = native.row_block_edges(b, m, 256)
             assert 8 <= edges <= cap[b] and edges % 4 == 0
+
+
+def test_rollout_tasks_cover_every_edge_once(lib):
+    """plan_rollout: each row's tasks take its edges h, h + slices, ... once, on
+    neighbouring lanes of one chunk from a multiple of `slices` on, within the quads
+    its wavefront holds; too many neurons or edges, or a row longer than a block, give
+    no plan."""
+    rng = np.random.default_rng(7)
+    for n, m, batch in ((1, 0, 1), (1, 7, 2), (40, 300, 4), (1024, 16_000, 1), (1024, 16_000, 8),
+                        (2048, 20_000, 16), (300, 4_000, 3)):
+        degree = rng.multinomial(m, np.full(n, 1.0 / n))
+        if n > 100:
+            degree[3], degree[5] = 0, degree[5] + (150 if batch < 16 else 20)
+        rowptr = np.concatenate([[0], np.cumsum(degree)]).astype(np.int32)
+        bounds = plan(lib, rowptr, native.row_block_edges(batch, int(rowptr[-1]), 256))
+        slots, tasks, rounds = native.plan_rollout(rowptr, bounds, batch)
+        seen = np.zeros(int(rowptr[-1]), np.int64)
+        rows = np.zeros(n, np.int64)
+        for wave in range(native.ROLLOUT_WAVES):
+            assert 4 * int((rounds[wave] & 0xFFFF).sum()) <= slots
+            for r, word in enumerate(rounds[wave]):
+                quads, slices = int(word) & 0xFFFF, 1 << (int(word) >> 16)
+                for lane, (first, packed) in enumerate(tasks[wave, r].tolist()):
+                    count, row = packed & 0xFFFF, (packed >> 16) & 0xFFFF
+                    if row == 0xFFFF:
+                        assert count == 0
+                        continue
+                    h = lane & (slices - 1)
+                    assert quads and count <= 4 * quads and first == rowptr[row] + h
+                    edges = first + slices * np.arange(count)
+                    assert np.all(edges < rowptr[row + 1]) and \
+                        (count == 0 or edges[-1] + slices >= rowptr[row + 1])
+                    seen[edges] += 1
+                    rows[row] += h == 0
+        assert np.all(seen == 1) and np.all(rows == 1)
+    even = lambda n, d: np.arange(n + 1, dtype=np.int32) * d  # noqa: E731
+    for n, d in ((2049, 1), (1024, 64)):
+        assert native.plan_rollout(even(n, d), plan(lib, even(n, d), 1024), 4) is None
+    hub = np.array([0, 3000, 3001], np.int32)
+    assert native.plan_rollout(hub, plan(lib, hub, 1024), 4) is None
+
+
+def test_rollout_validation_messages(lib):
+    """ns_dendritic_step with a rollout rejects bad arguments before any launch."""
+    n, batch = 8, 1
+    floats = (ctypes.c_float * 4096)()
+    base = ctypes.addressof(floats)
+    place = lambda k: base + 4 * 64 * k  # noqa: E731
+
+    def call(**fields):
+        args, rollout = native._StepArgs(), native._Rollout(4, 16, 1, 0)
+        rollout.tasks = rollout.rounds = place(40)
+        args.n_neurons, args.batch = n, batch
+        for i in range(6):
+            args.params[i] = native._Vector(place(30), 1)
+        args.matrix = native._Csr(n, 0, place(31), None, None, native.WEIGHT_F32, None, None)
+        for k, name in enumerate(("state", "dendrite", "adaptation")):
+            setattr(args, name, native._Plane(place(k), n, 1, 0.0))
+            setattr(args, "out_" + name, native._OutPlane(place(k), n, 1))
+        for name, value in fields.items():
+            setattr(rollout if hasattr(rollout, name) else args, name, value)
+        args.rollout = ctypes.addressof(rollout)
+        rc = lib.ns_dendritic_step(ctypes.byref(args), None)
+        return rc, lib.ns_last_error().decode()
+
+    for fields, text in (
+            ({"n_neurons": 2049, "matrix": native._Csr(2049, 0, place(31), None, None,
+                                                       native.WEIGHT_F32, None, None)},
+             "at most 2048"),
+            ({"ticks": 0}, "at least one tick"), ({"slots": 20}, "16, 32 or 48"),
+            ({"n_rounds": 8}, "1 to 7 rounds"), ({"tasks": None}, "tasks and rounds"),
+            ({"drive_tick": -1, "drive": native._Plane(place(20), n, 1, 0.0)}, "negative"),
+            ({"out_state": native._OutPlane(place(0), 0, 1), "batch": 2}, "overlap themselves"),
+            ({"out_state": native._OutPlane(place(1), n, 1)}, "overlap inputs"),
+            ({"trace": native._OutPlane(place(0), n, 1), "trace_tick": n}, "overlap"),
+            ({"out_current": native._OutPlane(place(9), n, 1)}, "no current")):
+        rc, message = call(**fields)
+        assert rc != 0 and text in message, (fields, message)

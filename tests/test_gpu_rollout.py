@@ -188,3 +188,58 @@ def _pad(values: torch.Tensor, ticks: int) -> torch.Tensor:
     out = torch.zeros((ticks, *values.shape[1:]), dtype=values.dtype)
     out[: values.shape[0]] = values
     return out
+
+
+@pytest.mark.parametrize("n,m,batch,fmt,staged", [
+    (1, 1, 1, None, False), (5, 3, 2, None, True), (200, 5_000, 3, "fp8", True),
+    (1024, 16_384, 4, None, True), (1024, 16_384, 1, "nvfp4", False),
+    (1023, 30_000, 2, "fp16", True), (1025, 9_000, 8, None, False),
+    (2048, 12_000, 16, "fp8", True), (2047, 30_000, 5, None, True), (700, 9_000, 17, None, False),
+    (1024, 30_000, 4, None, True)])
+def test_one_launch_rollout_is_bitwise_the_eager_ticks(gpu, n, m, batch, fmt, staged):
+    """Networks that fit a compute unit per column run a chunk in one launch
+    (ns_rollout): states and trace bitwise those of eager row-block ticks over two
+    chunks, with one or two neurons per lane, 16 to 48 edges per lane, empty rows and
+    rows of a whole block, every weight format, fixed and staged drives."""
+    print(f"case one-launch rollout N={n} M={m} B={batch} {fmt} staged={staged}", flush=True)
+    case = make_case(n, m, 3, gpu, kind="reference")
+    kwargs = ({} if fmt is None else {"weight_dtype": torch.float16} if fmt == "fp16"
+              else {"weight_format": fmt})
+    start = torch.rand(batch, n, generator=torch.Generator().manual_seed(n)).to(gpu)
+    eager, seeded = (NativeDendriticMatrixRuntime(case.topology, case.model, start.clone(),
+                                                  **kwargs) for _ in range(2))
+    ticks = 6
+    gen = torch.Generator().manual_seed(batch)
+    if staged:
+        soma = (torch.rand(ticks, batch, n, generator=gen) * 0.4).to(gpu)
+        dend = (torch.rand(ticks, batch, 1, generator=gen) * 0.2).to(gpu)
+    else:
+        soma, dend = column_drive(batch).to(gpu), 0.1
+    rollout = MatrixRollout(seeded, ticks, drive=soma, dendritic_drive=dend, trace=True)
+    assert rollout._resident is not None and rollout.graph is None
+    for chunk in range(2):
+        if chunk and staged:
+            soma = (torch.rand(ticks, batch, n, generator=gen) * 0.4).to(gpu)
+            rollout.stage(soma)
+        rollout.run()
+        for t in range(ticks):
+            eager.step(soma[t] if staged else soma,
+                       dendritic_drive=dend[t].expand(batch, n) if staged else dend)
+            assert torch.equal(rollout.trace[t], eager.state), (chunk, t)
+        for field in FIELDS:
+            assert torch.equal(getattr(rollout, field), getattr(eager, field)), (chunk, field)
+    rollout.advance(3)
+    for t in range(3):
+        eager.step(soma[t] if staged else soma,
+                   dendritic_drive=dend[t].expand(batch, n) if staged else dend)
+    for field in FIELDS:
+        assert torch.equal(getattr(rollout, field), getattr(eager, field)), field
+
+
+def test_rollouts_that_do_not_fit_use_the_graph(gpu):
+    for n, m, batch in ((2049, 4_000, 1), (1500, 90_000, 2), (300, 2_000, 300)):
+        case = make_case(n, m, 3, gpu)
+        runtime = NativeDendriticMatrixRuntime(case.topology, case.model,
+                                               torch.zeros(batch, n, device=gpu))
+        rollout = MatrixRollout(runtime, 2, drive=0.2)
+        assert rollout._resident is None and rollout.graph is not None
