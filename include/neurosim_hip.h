@@ -255,14 +255,17 @@ typedef struct ns_step_args {
  * wavefronts walks its chunks (`n_rounds` of them, the last ones possibly empty). */
 typedef struct ns_rollout {
   int32_t ticks;               /* > 0 */
-  int32_t slots;               /* edges per lane held in registers: 16, 32 or 48 */
+  int32_t slots;               /* edges per lane held in registers: 16, 32 or, up to 1024
+                                  neurons, 48 */
   int32_t n_rounds;            /* chunks per wavefront */
   int32_t reserved;
   const int32_t* tasks;        /* [16][n_rounds][64] pairs: first CSR edge; edge count in the
                                   low 16 bits and row in the high 16 (0xFFFF: no task) */
-  const int32_t* rounds;       /* [16][n_rounds]: quads of edges per lane (0: no chunk) in the
-                                  low 16 bits, log2 slices in the high 16; at most slots / 4
-                                  quads per wavefront */
+  const int32_t* rounds;       /* [16][n_rounds]: units of four slots per lane in the low 16
+                                  bits (0: no chunk), log2 slices in bits 16-18, and bit 31 if
+                                  the last unit is a tail: a lane's whole quads of edges come
+                                  first, the one to three edges left of every lane in that
+                                  unit.  At most slots / 4 units per wavefront */
   int64_t drive_tick;          /* floats from one tick's drive plane to the next (0: the same */
   int64_t dendritic_tick;      /* plane every tick) */
   ns_out_plane trace;          /* optional: s after each tick, [B,N] at trace.data + */

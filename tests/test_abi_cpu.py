@@ -619,14 +619,16 @@ def test_rollout_tasks_cover_every_edge_once(lib):
         for wave in range(native.ROLLOUT_WAVES):
             assert 4 * int((rounds[wave] & 0xFFFF).sum()) <= slots
             for r, word in enumerate(rounds[wave]):
-                quads, slices = int(word) & 0xFFFF, 1 << (int(word) >> 16)
+                units, slices = int(word) & 0xFFFF, 1 << ((int(word) >> 16) & 7)
+                quads = units - (int(word) < 0)            # bit 31: the last unit is a tail
                 for lane, (first, packed) in enumerate(tasks[wave, r].tolist()):
                     count, row = packed & 0xFFFF, (packed >> 16) & 0xFFFF
                     if row == 0xFFFF:
                         assert count == 0
                         continue
                     h = lane & (slices - 1)
-                    assert quads and count <= 4 * quads and first == rowptr[row] + h
+                    assert units and first == rowptr[row] + h
+                    assert count // 4 <= quads and (count % 4 == 0 or int(word) < 0)
                     edges = first + slices * np.arange(count)
                     assert np.all(edges < rowptr[row + 1]) and \
                         (count == 0 or edges[-1] + slices >= rowptr[row + 1])
