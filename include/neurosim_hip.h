@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define NS_ABI_VERSION 22
+#define NS_ABI_VERSION 23
 
 /* Return codes. */
 #define NS_OK 0
@@ -410,7 +410,14 @@ typedef struct ns_step_grad_args {
                                   then unused.  Its partials workspace must not overlap
                                   the gradient planes or the workspace. */
   int32_t flags;               /* NS_GRAD_* */
-  int32_t reserved;
+  int32_t pending_entry;       /* 0 or 1, with `pending` */
+  float* pending;              /* optional float32[2][N][2*B]: what the weight gradients of two
+                                  ticks are made of, the gradients of j (first N*2B floats) and
+                                  the states, entry e of neuron n in columns e*B to e*B + B.
+                                  This tick's are stored as entry `pending_entry`, and the
+                                  weight gradient is left to the call that stores entry 1: it
+                                  gives d_weight both ticks' in one pass over the edges
+                                  (`d_weight` must be NULL with entry 0). */
 } ns_step_grad_args;
 
 /* ns_step_grad_args flag: the caller does not want the gradient of the state

@@ -41,6 +41,7 @@ struct GradArgs {
   float* gj;             // [N][B]
   float* gp[6];
   int32_t add_params;    // add to gp instead of storing
+  OutPlane pg, ps;       // optional copies of gj and s (the pending entry)
 };
 
 // One lane per (neuron, column), LB lanes per neuron; lane q takes columns q,
@@ -90,7 +91,12 @@ __global__ __launch_bounds__(kGradThreads) void advance_backward_kernel(GradArgs
     A.ga.put(b, n, P.rho_a * gA - P.strength * g_x2);
     if (A.gu.data) A.gu.put(b, n, g_x2);
     if (A.gv.data) A.gv.put(b, n, g_x1);
-    A.gj[n * A.B + b] = (1.0f - P.coupling) * g_x2 + g_x1;
+    const float g_j = (1.0f - P.coupling) * g_x2 + g_x1;
+    A.gj[n * A.B + b] = g_j;
+    if (A.pg.data) {
+      A.pg.put(b, n, g_j);
+      A.ps.put(b, n, s);
+    }
   }
   float sums[6] = {g_alpha, g_gain, g_rho_d, g_rho_a, g_c, g_k};
 #pragma unroll
@@ -255,6 +261,11 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
   if (a.transposed_panels && batch > 2) return fail("transposed panels need batch 1 or 2");
   if (a.flags & ~(NS_GRAD_NO_STATE | NS_GRAD_ADD_WEIGHT | NS_GRAD_ADD_PARAMS)) return fail("unknown backward flags %d", a.flags);
   const bool want_state = (a.flags & NS_GRAD_NO_STATE) == 0;
+  if (a.pending) {
+    if (a.pending_entry != 0 && a.pending_entry != 1) return fail("a pending entry is 0 or 1");
+    if (a.pending_entry == 0 && a.d_weight)
+      return fail("the weight gradient comes with pending entry 1");
+  }
   const Extent outs[5] = {extent(a.d_state, batch, n), extent(a.d_dendrite, batch, n),
                           extent(a.d_adaptation, batch, n), extent(a.d_drive, batch, n),
                           extent(a.d_dendritic_drive, batch, n)};
@@ -264,6 +275,12 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
                          extent(a.grad_dendrite, batch, n), extent(a.grad_adaptation, batch, n),
                          extent_of(a.current, 1, 1, 1, batch * n)};
   const Extent work = extent_of(a.workspace, 1, 1, 1, 2 * batch * n);
+  const Extent pending = extent_of(a.pending, 1, 1, 1, 4 * batch * n);
+  if (overlaps(pending, work)) return fail("the pending entries must not overlap the workspace");
+  for (const Extent& in : ins)
+    if (overlaps(pending, in)) return fail("the pending entries must not overlap inputs");
+  for (const Extent& out : outs)
+    if (overlaps(pending, out)) return fail("the pending entries must not overlap gradient planes");
   if (overlaps(ins[8], work)) return fail("the forward's current must not overlap the workspace");
   for (int o = 0; o < 5; ++o) {
     if (overlaps(outs[o], work)) return fail("gradient planes must not overlap the workspace");
@@ -300,6 +317,11 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
   G.gj = gj;
   for (int i = 0; i < 6; ++i) G.gp[i] = a.d_params[i];
   G.add_params = (a.flags & NS_GRAD_ADD_PARAMS) != 0;
+  if (a.pending) {
+    float* const entry = a.pending + a.pending_entry * batch;
+    G.pg = OutPlane{entry, 1, 2 * batch};
+    G.ps = OutPlane{entry + 2 * batch * n, 1, 2 * batch};
+  }
   // The transposed product on panels: W^T @ gj added into d_state.
   ns_step_args transposed{};
   if (want_state && a.transposed_panels && a.matrix.n_edges > 0) {
@@ -347,15 +369,24 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
       });
     }
     if (a.d_weight) {
-      // The state's rows load whole when it is neuron-major and aligned too.
-      const int64_t width = batch % 4 == 0 ? 4 : 2;
-      const bool s_rows = gj_rows && a.state.stride_b == 1 && a.state.stride_n % width == 0 &&
-                          reinterpret_cast<uintptr_t>(a.state.data) % (4 * width) == 0;
-      const EdgeForm form = edge_form(batch, s_rows);
+      // One tick's columns, or the two pending ticks' side by side: the gather of an
+      // edge is one request either way, and the pass is bound by those and by the
+      // edges' indices and gradients (N=166k, M=25M, B=1: 131 us for one tick,
+      // 136 for two).
+      const int64_t cols = a.pending ? 2 * batch : batch;
+      const float* const g = a.pending ? a.pending : gj;
+      const Plane from = a.pending ? Plane{a.pending + 2 * batch * n, 1, cols, 0.0f, ~0u}
+                                   : plane(a.state, a.state.data);
+      // Rows load whole where they are neuron-major and aligned.
+      const int64_t width = cols % 4 == 0 ? 4 : 2;
+      const bool whole = cols % width == 0 && from.sb == 1 && from.sn % width == 0 &&
+                         reinterpret_cast<uintptr_t>(from.data) % (4 * width) == 0 &&
+                         reinterpret_cast<uintptr_t>(g) % (4 * width) == 0;
+      const EdgeForm form = edge_form(cols, whole);
       const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe);
       with_edge_form(form, [&](auto vl, auto lpe) {
         weight_gradient_kernel<vl(), lpe()><<<lanes_grid(n, form.lpe << lg), kGradThreads, 0, s>>>(
-            a.matrix.rowptr, a.matrix.col, gj, plane(a.state, a.state.data), n, batch, a.d_weight,
+            a.matrix.rowptr, a.matrix.col, g, from, n, cols, a.d_weight,
             (a.flags & NS_GRAD_ADD_WEIGHT) != 0, lg);
       });
     }

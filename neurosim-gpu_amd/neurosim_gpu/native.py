@@ -37,7 +37,7 @@ import numpy as np
 import torch
 
 _LIB_NAME = "libneurosim_hip.so"
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 WEIGHT_F32, WEIGHT_F16, WEIGHT_E4M3, WEIGHT_NVFP4 = 0, 1, 2, 3
 _PLAN_CACHE = 64   # row plans kept per extension (one per live topology and batch width)
@@ -152,7 +152,8 @@ class _StepGradArgs(ctypes.Structure):
                 ("d_drive", _OutPlane), ("d_dendritic_drive", _OutPlane),
                 ("d_weight", _c_ptr), ("d_params", _c_ptr * 6), ("workspace", _c_ptr),
                 ("current", _c_ptr), ("out_weight", _c_ptr), ("transposed_panels", _c_ptr),
-                ("flags", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+                ("flags", ctypes.c_int32), ("pending_entry", ctypes.c_int32),
+                ("pending", _c_ptr)]
 
 GRAD_NO_STATE, GRAD_ADD_WEIGHT, GRAD_ADD_PARAMS = 1, 2, 4   # NS_GRAD_*
 
@@ -1426,7 +1427,9 @@ class PreparedBackward:
     is then the update's own part, for a caller that drops it.  ``sums`` gives the
     weight gradient and the parameter gradients' block of later ticks, which this
     tick's are added to in place (as autograd would add them, in the same order).
-    Last of the results is the parameter gradients' block; ``split=False`` leaves
+    ``pending`` ([2, N, 2B]) defers the weight gradient: a call with
+    ``pending_entry`` 0 only stores what its own is made of, the next one, with 1, gives
+    both ticks' in one pass.  Last of the results is the parameter gradients' block; ``split=False`` leaves
     out the list of its rows."""
 
     def __init__(self, extension: "NativeExtension", state: torch.Tensor, params, rowptr, col,
@@ -1471,7 +1474,8 @@ class PreparedBackward:
                  dendritic_scalar, grad_state, grad_dendrite, grad_adaptation, *,
                  need_drive=False, need_dendritic=False, need_weight=False,
                  need_params=(False,) * 6, out_weight=None, current=None,
-                 transposed_panels=None, need_state=True, sums=(None, None), split=True):
+                 transposed_panels=None, need_state=True, sums=(None, None), split=True,
+                 pending=None, pending_entry=0):
         _check_state(state)
         if state.device != self.device:
             raise RuntimeError("all tensors must be on the state's CUDA device")
@@ -1518,7 +1522,7 @@ class PreparedBackward:
             if d_weight.shape != weight.shape or not d_weight.is_contiguous():
                 raise RuntimeError("the weight gradient must be a contiguous [M] vector")
             flags |= GRAD_ADD_WEIGHT
-        elif need_weight:
+        elif need_weight and not (pending is not None and pending_entry == 0):
             d_weight = torch.empty(weight.shape, dtype=torch.float32, device=self.device)
         wanted = [i for i, want in enumerate(need_params) if want]
         work = self._work
@@ -1537,8 +1541,16 @@ class PreparedBackward:
         param_ptrs = [0] * 6
         for k, i in enumerate(wanted):
             param_ptrs[i] = start + 4 * k * n
-        _POINTERS11.pack_into(args, _GRAD_POINTERS,
-                              d_weight.data_ptr() if d_weight is not None and weight.numel() else 0,
+        args.pending = None
+        weight_ptr = d_weight.data_ptr() if d_weight is not None and weight.numel() else 0
+        if pending is not None:
+            _check_float(pending, state, "pending entries")
+            if pending.shape != (2, n, 2 * batch) or not pending.is_contiguous():
+                raise RuntimeError("pending entries must be a contiguous [2, N, 2B] block")
+            args.pending, args.pending_entry = pending.data_ptr(), pending_entry
+            if pending_entry == 0:       # sums pass by unchanged
+                weight_ptr, flags = 0, flags & ~GRAD_ADD_WEIGHT
+        _POINTERS11.pack_into(args, _GRAD_POINTERS, weight_ptr,
                               *param_ptrs, workspace.data_ptr() if work else 0, current_ptr,
                               out_weight_ptr,
                               ctypes.addressof(transposed_panels) if transposed_panels is not None

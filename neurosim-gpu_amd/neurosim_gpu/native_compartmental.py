@@ -223,12 +223,15 @@ class _Recording:
     returned, on the same weights and parameters.
 
     Only its first tick takes the weights and parameters as autograd inputs.
-    Every tick also returns two tokens, zero-stride tensors of the shapes of the
-    weight gradient and of the parameter gradients' block, and takes those of the
-    tick before.  The gradient of a token is the sum of the later ticks'
-    gradients, which a tick's backward adds its own to in place and hands on, so
-    a backward through T ticks adds no pair of gradients outside the kernels
-    (seven torch additions per tick otherwise).  The states are held weakly:
+    Every tick also returns three tokens, zero-stride tensors of the shapes of the
+    weight gradient, of the parameter gradients' block and of a pair of pending
+    entries (ns_step_grad_args.pending), and takes those of the tick before.  The
+    gradients of the first two are the sums of the later ticks' gradients, which a
+    tick's backward adds its own to in place and hands on, so a backward through T
+    ticks adds no pair of gradients outside the kernels (seven torch additions per
+    tick otherwise).  The gradient of the third, when there is one, is the entry of
+    the tick after, whose weight gradient this tick's pass over the edges computes
+    together with its own.  The states are held weakly:
     once the caller drops them the tokens, and the graph behind them, go too."""
 
     __slots__ = ("states", "weight", "params", "versions", "topology", "stream", "tokens")
@@ -276,12 +279,15 @@ class _NativeTick(torch.autograd.Function):
         ctx.set_materialize_grads(False)
         ctx.wants = (weight.requires_grad, tuple(p.requires_grad for p in params))
         zero = state.new_empty(1)
+        batch, n = state.shape
         tokens = (zero.expand(weight.numel()) if ctx.wants[0] else None,
-                  zero.expand(sum(ctx.wants[1]) * state.shape[1]) if any(ctx.wants[1]) else None)
+                  zero.expand(sum(ctx.wants[1]) * n) if any(ctx.wants[1]) else None,
+                  zero.expand(2, n, 2 * batch) if ctx.wants[0] else None)
         return (*outs, *tokens)
 
     @staticmethod
-    def backward(ctx, grad_state, grad_dendrite, grad_adaptation, sum_weight, sum_params):
+    def backward(ctx, grad_state, grad_dendrite, grad_adaptation, sum_weight, sum_params,
+                 pending):
         info = ctx.info
         topology = info.topology
         saved = list(ctx.saved_tensors)
@@ -304,15 +310,22 @@ class _NativeTick(torch.autograd.Function):
         prepared = cache[0]
         if prepared is None or not prepared.matches(state, params, *fixed):
             prepared = cache[0] = PreparedBackward(info.extension, state, params, *fixed)
+        # The last tick of a pair leaves its weight gradient to the one before.
+        entry = 0 if pending is None else 1
+        if pending is None and need_weight and not info.first:
+            batch, n = state.shape
+            pending = torch.empty((2, n, 2 * batch), dtype=torch.float32, device=state.device)
         (d_state, d_dendrite, d_adaptation, d_drive, d_dendritic, d_weight, d_params,
          block) = prepared(
             state, dendrite, adaptation, drive, info.us, dendritic_drive, info.vs, grad_state,
             grad_dendrite, grad_adaptation, need_drive=bool(needs[4]),
             need_dendritic=bool(needs[5]), need_weight=need_weight, need_params=need_params,
             out_weight=out_weight, current=ctx.current, transposed_panels=panels,
-            need_state=bool(needs[1]), sums=(sum_weight, sum_params), split=info.first)
+            need_state=bool(needs[1]), sums=(sum_weight, sum_params), split=info.first,
+            pending=pending, pending_entry=entry)
         ctx.current = None
-        linked = (d_weight, *d_params) if info.first else (d_weight, block)
+        linked = ((d_weight, *d_params) if info.first
+                  else (d_weight, block, pending if entry == 0 else None))
         return (None, d_state if needs[1] else None, d_dendrite if needs[2] else None,
                 d_adaptation if needs[3] else None, d_drive, d_dendritic, *linked)
 
@@ -688,9 +701,10 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
                          prepared=self._prepared_backward, by_neuron=by_neuron, weight=weight,
                          params=params, first=first)
         linked = (weight, *params) if first else recording.tokens
-        *states, token_weight, token_params = _NativeTick.apply(info, *states, u, v, *linked)
+        s, d, a, *tokens = _NativeTick.apply(info, *states, u, v, *linked)
+        states = (s, d, a)
         self._recording = _Recording(states, weight, params, versions, topology, stream,
-                                     (token_weight, token_params))
+                                     tuple(tokens))
         self.state, self.dendritic_state, self.adaptation_state = states
         self.last_backend = "native-autograd"
         return self.state

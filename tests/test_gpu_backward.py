@@ -369,7 +369,8 @@ def test_gradients_summed_through_the_ticks_equal_separate_ones(gpu, batch, kern
     tick, each backward adding to them in place.  Against ticks recorded one by one
     (autograd adds their gradients, in the same order): bitwise, also through a second
     backward of the same graph, with some parameters frozen, and for a loss that leaves
-    out the last ticks."""
+    out the last ticks (the weight gradient to float32 rounding: it comes two ticks at
+    a time)."""
     print(f"case backward linked ticks batch={batch} kernel={kernel}", flush=True)
     g = graph(900, 20_000, 8)
     inputs = inputs_for(g, batch, 50 + batch)
@@ -399,8 +400,15 @@ def test_gradients_summed_through_the_ticks_equal_separate_ones(gpu, batch, kern
         for early in (False, True):
             one, again = gradients(True, frozen, early)
             separate, _ = gradients(False, frozen, early)
-            for a, b, c in zip(one, separate, again):
-                assert torch.equal(a, b)
+            for k, (a, b, c) in enumerate(zip(one, separate, again)):
+                if k == 0:
+                    # Two ticks' weight gradients come from one chain of fused multiply-adds
+                    # over 2B columns instead of two chains and an addition: at most two
+                    # roundings of the partial sums (below twice the largest gradient) per term.
+                    assert float((a - b).abs().max()) <= 8 * batch * 2.0 ** -23 * \
+                        float(a.abs().max())
+                else:
+                    assert torch.equal(a, b)
                 # the second backward recomputes j = W @ s on row blocks
                 assert float((a - c).abs().max()) <= 1e-5 * float(a.abs().max())
 
