@@ -164,6 +164,15 @@ class _EncodeArgs(ctypes.Structure):
                 ("global_scale", _c_ptr), ("workspace", _c_ptr)]
 
 
+class _BlockedPermutation(ctypes.Structure):
+    _fields_ = [("n_edges", _c_i64), ("n_slots", _c_i64), ("chunk", ctypes.c_int32),
+                ("bucket", ctypes.c_int32), ("n_chunks", ctypes.c_int32),
+                ("n_buckets", ctypes.c_int32), ("place", _c_ptr), ("run_start", _c_ptr),
+                ("run_target", _c_ptr), ("bucket_start", _c_ptr), ("slot_source", _c_ptr)]
+
+BLOCKED_MAX = 36_864   # NS_BLOCKED_MAX (neurosim_hip_layout.h)
+
+
 class _TopologyArgs(ctypes.Structure):
     _fields_ = [("n_neurons", _c_i64), ("n_candidates", _c_i64), ("src", _c_ptr),
                 ("dst", _c_ptr), ("weight", _c_ptr), ("out_src", _c_ptr), ("out_dst", _c_ptr),
@@ -206,6 +215,8 @@ def load_library() -> ctypes.CDLL:
     lib.ns_gather_slot_weights.restype = ctypes.c_int
     lib.ns_gather_slot_weights.argtypes = [_c_ptr, _c_i64, _c_i64, ctypes.c_int32, ctypes.c_int32,
                                            _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr]
+    lib.ns_permute_blocked.restype = ctypes.c_int
+    lib.ns_permute_blocked.argtypes = [ctypes.POINTER(_BlockedPermutation)] + [_c_ptr] * 4
     lib.ns_plan_bands.restype = ctypes.c_int
     lib.ns_plan_bands.argtypes = [_c_ptr, _c_ptr, _c_i64, ctypes.c_int32, ctypes.c_int32,
                                   ctypes.c_int32, ctypes.POINTER(_BandPlan)] + [_c_ptr] * 5
@@ -532,6 +543,7 @@ class _SlotLayout:
     n_slots: int
     perm: torch.Tensor
     pairs: bool = False
+    blocked: "BlockedPermutation | None" = None    # float32 weights in two streaming passes
     _slot_weights: tuple | None = None
     _slot_key = None
 
@@ -541,6 +553,10 @@ class _SlotLayout:
             return self._slot_weights
         device, n = weight.device, self.n_slots
         nvfp4 = block_scales is not None
+        if self.blocked is not None and not nvfp4 and weight.dtype == torch.float32:
+            self._slot_weights = (self.blocked(weight.detach()), None)
+            self._slot_key = key
+            return self._slot_weights
         if not nvfp4:
             fmt = {torch.float32: WEIGHT_F32, torch.float16: WEIGHT_F16,
                    torch.uint8: WEIGHT_E4M3}[weight.dtype]
@@ -566,6 +582,66 @@ class _SlotLayout:
         self._slot_weights = (slots, scales)
         self._slot_key = key
         return self._slot_weights
+
+
+class BlockedPermutation:
+    """The tables of ns_permute_blocked for a slot permutation ``perm`` (int32 on the
+    device: each slot's edge, every edge in one slot, -1 for padding)."""
+
+    def __init__(self, perm: torch.Tensor, n_edges: int, chunk: int | None = None,
+                 bucket: int | None = None) -> None:
+        # us per call (chunk / bucket) on transposed panel layouts: 25M edges 128 at
+        # 18432 / 18432, 120 at 18432 / 36864, 220 at 9216 / 9216; 10M 48, 58, 59; 4M
+        # 29, 36, 25; slot by slot (ns_gather_slot_weights) 418, 148 and 57.
+        half = BLOCKED_MAX // 2
+        chunk = chunk or (half if n_edges >= 6_000_000 else half // 2)
+        bucket = bucket or (BLOCKED_MAX if n_edges >= 20_000_000 else chunk)
+        device, n_slots = perm.device, perm.numel()
+        chunks = -(-n_edges // chunk)
+        buckets = -(-n_slots // bucket)
+        slots = torch.nonzero(perm >= 0).view(-1).to(torch.int32)
+        if slots.numel() != n_edges:
+            raise RuntimeError("a blocked permutation holds every edge in one slot")
+        slot_of = torch.empty(n_edges, dtype=torch.int32, device=device)
+        slot_of[perm[slots].long()] = slots
+        edge = torch.arange(n_edges, dtype=torch.int32, device=device)
+        # Runs: (chunk, bucket), the chunk's edges of one bucket, in edge order.
+        run = (edge // chunk) * buckets + slot_of // bucket
+        order = torch.sort(run, stable=True).indices
+        place = torch.empty_like(edge)
+        place[order] = edge                       # position among all chunks' runs
+        counts = torch.bincount(run, minlength=chunks * buckets).view(chunks, buckets)
+        starts = torch.zeros(chunks, buckets + 1, dtype=torch.int64, device=device)
+        starts[:, 1:] = counts.cumsum(1)
+        by_bucket = counts.t().reshape(-1).cumsum(0)          # bucket-major, inclusive
+        targets = (by_bucket - counts.t().reshape(-1)).view(buckets, chunks).t().contiguous()
+        bucket_start = torch.zeros(buckets + 1, dtype=torch.int64, device=device)
+        bucket_start[1:] = by_bucket.view(buckets, chunks)[:, -1] if chunks else 0
+        place -= (edge // chunk) * chunk
+        # Where each edge's value lies within its bucket's values.
+        within = (targets.view(-1)[run.long()] - bucket_start[(slot_of // bucket).long()]
+                  + place - starts[:, :-1].reshape(-1)[run.long()])
+        source = torch.full((n_slots,), -1, dtype=torch.int16, device=device)
+        source[slot_of.long()] = within.to(torch.int16)       # uint16 bits
+        self._tables = (place.to(torch.int16), starts.to(torch.int16).contiguous(),
+                        targets.to(torch.int32), bucket_start.to(torch.int32), source)
+        self._args = _BlockedPermutation(n_edges, n_slots, chunk, bucket, chunks, buckets,
+                                         *(t.data_ptr() if t.numel() else None
+                                           for t in self._tables))
+
+    def __call__(self, values: torch.Tensor) -> torch.Tensor:
+        """``values`` (float32 [M], contiguous) in slot order, padding zero."""
+        args = self._args
+        if (values.dtype != torch.float32 or values.shape != (args.n_edges,)
+                or not values.is_contiguous() or values.device != self._tables[0].device):
+            raise RuntimeError("the values must be M contiguous float32 on the layout's device")
+        slots = torch.empty(args.n_slots, dtype=torch.float32, device=values.device)
+        workspace = torch.empty(max(args.n_edges, 4), dtype=torch.float32, device=values.device)
+        lib = load_library()
+        _raise_on(lib.ns_permute_blocked(
+            ctypes.byref(args), values.data_ptr() if args.n_edges else None, workspace.data_ptr(),
+            slots.data_ptr(), ctypes.c_void_p(current_stream(values.device))), lib)
+        return slots
 
 
 class PanelLayout(_SlotLayout):

@@ -32,6 +32,7 @@ import torch
 
 from .compartmental import DendriticDynamics, DendriticMatrixRuntime, DendriticPELSRuntime
 from .native import (BAND_WIDTH, EVENT_ACTIVITY_SLOTS, EVENT_ACTIVITY_STRIDE, BandLayout,
+                     BlockedPermutation,
                      NativeExtension, PanelLayout, PreparedAccumulate, PreparedBackward,
                      PreparedEvent, PreparedTick, _neuron_major, current_stream, encode_weights,
                      load_native_extension, new_planes, panel_geometry)
@@ -150,6 +151,12 @@ class SourceMajorWeights:
         return self._values
 
 
+# Fewest edges for which the transposed weights are permuted in two streaming passes
+# before their first use.  us per product on new weights, indexed / copy + streamed:
+# 4M edges, B=1 37 / 25 + 13; 10M, B=2 107 / 48 + 27; 25M, B=1 334 / 120 + 33.
+BLOCKED_MIN_EDGES = 4_000_000
+
+
 class TransposedPanels:
     """Column-panel layout of the transposed matrix, for the backward's W^T @ g.
 
@@ -161,9 +168,10 @@ class TransposedPanels:
     The slot-order copy, one random read per edge, is made on the first request
     when ``expect`` has announced two or more products of the version
     (backpropagation through several ticks), else on the second (repeated passes
-    on fixed weights), and streamed after that.  N=166k, M=25M: an indexed
-    product takes 327 us, the copy 413 and a streamed product 33, so two
-    products cost 479 us with the copy made at once and 773 with it made late.
+    on fixed weights), and streamed after that.  From ``BLOCKED_MIN_EDGES`` edges
+    on the copy is made at once: two streaming passes (``BlockedPermutation``) cost
+    less than the indexed product's reads (N=166k, M=25M: copy 120 us and streamed
+    product 33 against 334 indexed; slot by slot the copy took 418).
     Built on the host from the source-major view (set-up only, like the
     forward's layout)."""
 
@@ -176,6 +184,8 @@ class TransposedPanels:
         owi = topology.out_weight_index.to(device=device, dtype=torch.int32)
         self.layout.perm = torch.where(perm >= 0, owi[perm.clamp(min=0).long()],
                                        perm).to(torch.int32).contiguous()
+        if topology.n_edges >= BLOCKED_MIN_EDGES:
+            self.layout.blocked = BlockedPermutation(self.layout.perm, topology.n_edges)
         self._key, self._source, self._seen, self._expected = None, None, 0, 0
         self._indexed = None
 
@@ -198,8 +208,8 @@ class TransposedPanels:
         key = self._version(weight)
         self._seen += 1
         # No copy inside a capture: it would be filled only when the graph replays.
-        if (self._seen < 2 and self._expected < 2) or (
-                self.layout._slot_key != key and torch.cuda.is_current_stream_capturing()):
+        late = self.layout.blocked is None and self._seen < 2 and self._expected < 2
+        if late or (self.layout._slot_key != key and torch.cuda.is_current_stream_capturing()):
             if self._indexed is None:
                 self._indexed = self.layout.indexed_plan_struct()
             return self._indexed

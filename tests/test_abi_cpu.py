@@ -678,3 +678,28 @@ def test_rollout_validation_messages(lib):
             ({"out_current": native._OutPlane(place(9), n, 1)}, "no current")):
         rc, message = call(**fields)
         assert rc != 0 and text in message, (fields, message)
+
+
+def test_blocked_permutation_validation_messages(lib):
+    """ns_permute_blocked rejects bad arguments before any launch."""
+    base = ctypes.addressof((ctypes.c_float * 4096)())
+    base += -base % 16
+
+    def call(**fields):
+        given = dict(n_edges=100, n_slots=128, chunk=64, bucket=64, n_chunks=2, n_buckets=2,
+                     place=base, run_start=base, run_target=base, bucket_start=base,
+                     slot_source=base)
+        slots = fields.pop("slots", base + 4096)
+        given.update(fields)
+        args = native._BlockedPermutation(**given)
+        rc = lib.ns_permute_blocked(ctypes.byref(args), base, base + 2048, slots, None)
+        return rc, lib.ns_last_error().decode()
+
+    for fields, text in (({"n_slots": 126}, "multiple of 4"), ({"chunk": 6}, "multiple of 4 from"),
+                         ({"bucket": 36_868}, "to 36864"), ({"n_chunks": 3}, "chunks for 100"),
+                         ({"n_buckets": 1}, "buckets for 128"), ({"place": None}, "chunk tables"),
+                         ({"slot_source": None}, "tables, workspace"),
+                         ({"slots": base + 4100}, "16-byte"), ({"slots": base + 2048}, "overlap")):
+        rc, message = call(**fields)
+        assert rc != 0 and text in message, (fields, message)
+    assert call(n_slots=0, n_buckets=0)[0] == 0

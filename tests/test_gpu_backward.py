@@ -450,3 +450,54 @@ def test_a_run_of_recorded_ticks_ends_where_its_inputs_change(gpu):
     for a, b in zip(gradients(True), gradients(False)):
         # branches meet in another order of additions: a few roundings of the sum
         assert float((a - b).abs().max()) <= 2.0 ** -20 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("n,m,chunk,bucket", [
+    (50, 400, None, None), (3000, 90_000, None, None), (3000, 90_000, 4, 64),
+    (700, 9_217, 9216, 128), (2000, 60_000, 36_864, 36_864), (300, 5_001, 4_996, 18_432)])
+def test_blocked_permutation_equals_the_slot_gather(gpu, n, m, chunk, bucket):
+    """ns_permute_blocked (through LDS, chunk by chunk and bucket by bucket) against the
+    gather slot by slot, bitwise: chunks and buckets of a few values, partial last ones,
+    and values at an address that is not 16-byte aligned."""
+    print(f"case blocked permutation n={n} m={m} chunk={chunk} bucket={bucket}", flush=True)
+    from neurosim_gpu.native import BlockedPermutation
+    from neurosim_gpu.native_compartmental import TransposedPanels
+
+    topo = topology(graph(n, m, 3), torch.float32, gpu)
+    layout = TransposedPanels(topo, 1, gpu).layout
+    permutation = BlockedPermutation(layout.perm, topo.n_edges, chunk, bucket)
+    for offset in (0, 1):
+        held = torch.randn(topo.n_edges + offset, device=gpu)
+        values = held[offset:]
+        want, _ = layout.slot_weights(object(), values, None)
+        assert torch.equal(permutation(values), want)
+    with pytest.raises(RuntimeError, match="M contiguous float32"):
+        permutation(held[: topo.n_edges - 1])
+
+
+def test_blocked_transposed_weights_change_no_gradient(gpu, monkeypatch):
+    """Two weight versions through two ticks each, with the transposed weights permuted
+    in blocks before their first use: gradients bitwise those of the indexed plan."""
+    print("case backward blocked transposed weights", flush=True)
+    from neurosim_gpu import native_compartmental as nc
+
+    g = graph(3000, 90_000, 17)
+    inputs = inputs_for(g, 1, 77)
+    kw = dict(scalar_drives=False, expanded=False, kernel="panels", panel_width=1000)
+    indexed, rt = run(NativeDendriticMatrixRuntime, g, inputs, torch.float32, gpu, 1, **kw)
+    assert rt._transposed.layout.blocked is None
+    monkeypatch.setattr(nc, "BLOCKED_MIN_EDGES", 0)
+    blocked, rt = run(NativeDendriticMatrixRuntime, g, inputs, torch.float32, gpu, 1, **kw)
+    assert rt._transposed.layout.blocked is not None
+    assert rt._transposed.layout._slot_weights is not None
+    for name in indexed:
+        assert torch.equal(indexed[name], blocked[name]), name
+    with torch.no_grad():
+        rt.topology.in_weight.mul_(0.5)
+    before = rt._transposed.layout._slot_key
+    rt.state = rt.state.detach().requires_grad_(True)
+    rt.dendritic_state, rt.adaptation_state = (rt.dendritic_state.detach(),
+                                               rt.adaptation_state.detach())
+    rt.step(0.2)
+    rt.state.sum().backward()
+    assert rt._transposed.layout._slot_key != before
