@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 
 #include "ns_common.h"
 #include "ns_host.h"
@@ -44,8 +45,6 @@ template <>
 struct TileCfg<4> { static constexpr int passes = 1; };
 template <>
 struct TileCfg<8> { static constexpr int passes = 1; };
-template <>
-struct TileCfg<16> { static constexpr int passes = 1; };
 
 template <int BT>
 constexpr int block_capacity() { return kThreads * 4 * TileCfg<BT>::passes; }
@@ -64,7 +63,7 @@ struct TickArgs {
   OutPlane os, od, oa;
   OutPlane oj;          // optional: j as well (data null: not written)
   int32_t quad_loads;   // col/weight pointers aligned for one-quad vector loads
-  int32_t s_vec4;       // s is neuron-major with 16-byte aligned column groups
+  int32_t s_rows;       // s is neuron-major: a source's columns are neighbours
   int32_t spmm_only;    // write j to `os` instead of advancing
   int32_t spmm_accumulate;  // with spmm_only: add j to `os` instead
 };
@@ -163,11 +162,127 @@ __device__ void rows_one_by_one(const TickArgs& A, int r0, int r1, int b0, float
   }
 }
 
+// Lanes that share a source's row, each loading up to four of the tile's columns.
+template <int BT>
+constexpr int kShare = BT > 4 ? BT / 4 : 1;
+
+// Padded [column][edge] rows of a workgroup's products in LDS (16-byte aligned).
+template <int BT>
+constexpr int kProductStride = block_capacity<BT>() + 4;
+
+// The value of the first (k = 0) or second lane of this lane's pair (kLanes 2).
+template <int kLanes, int k>
+__device__ __forceinline__ int shared_lane(int x) {
+  if constexpr (kLanes == 1) return x;
+  constexpr int control = k == 0 ? 0xA0 : 0xF5;   // quad_perm 0 0 2 2 or 1 1 3 3
+  return __builtin_amdgcn_update_dpp(0, x, control, 0xF, 0xF, true);
+}
+
+// kCols neighbouring floats at any 4-byte aligned address, in one load.
+template <int kCols>
+__device__ __forceinline__ void load_columns(const float* at, float (&x)[4]) {
+  if constexpr (kCols == 1) {
+    x[0] = *at;
+  } else {
+    typedef float vec __attribute__((ext_vector_type(kCols)));
+    struct __attribute__((packed, aligned(4))) words { vec v; };
+    const vec y = reinterpret_cast<const words*>(at)->v;
+#pragma unroll
+    for (int k = 0; k < kCols; ++k) x[k] = y[k];
+  }
+}
+
+template <int BT, int kCols>
+__device__ __forceinline__ void gather_columns(const float* s, int64_t sn,
+                                               const int (&c)[4 * kShare<BT>], int first, int e0,
+                                               int e1, float (&g)[4 * kShare<BT>][4]) {
+#pragma unroll
+  for (int i = 0; i < 4 * kShare<BT>; ++i)
+    if (first + i >= e0 && first + i < e1) load_columns<kCols>(s + c[i] * sn, g[i]);
+}
+
+// Phase 1 of one pass for a neuron-major state.  At eight columns the two lanes of
+// a pair take their eight edges together, each loading four columns of every edge's
+// source row, so that one load instruction reads 32 whole rows and the L2 sees one
+// request per row rather than two (the lanes trade column indices and weights by
+// DPP).  A row needs 4-byte alignment only, so odd batches load the same way, in
+// one or two loads per edge where they took one per column.  The products and their
+// LDS places are those of the per-lane path, so the sums are bitwise the same.  us
+// per tick, N=50k, M=1M, fp32, before and after: B=2 10.5, 9.2; B=3 12.6, 10.0; B=5
+// 18.8, 13.9; B=7 23.9, 14.7; B=4 and 8 unchanged (9.9, 13.8).
+template <int BT, bool kWhole>
+__device__ __forceinline__ void gather_rows(const TickArgs& A, const int (&c_own)[4],
+                                            const float (&w_own)[4], bool have, int first, int e0,
+                                            int e1, int b0, float* prod) {
+  constexpr int kEdges = 4 * kShare<BT>;
+  constexpr int kWidth = BT < 4 ? BT : 4;
+  const int part = threadIdx.x & (kShare<BT> - 1);
+  const int cols = kWhole ? kWidth
+                          : static_cast<int>(min<int64_t>(kWidth, A.B - (b0 + kWidth * part)));
+  int c[kEdges];
+  float w[kEdges];
+  const auto trade = [&](auto lane) {
+    constexpr int k = decltype(lane)::value;
+    if constexpr (k < kShare<BT>) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        c[4 * k + j] = shared_lane<kShare<BT>, k>(have ? c_own[j] : 0);
+        w[4 * k + j] = __builtin_bit_cast(
+            float, shared_lane<kShare<BT>, k>(__builtin_bit_cast(int, have ? w_own[j] : 0.0f)));
+      }
+    }
+  };
+  trade(std::integral_constant<int, 0>{});
+  trade(std::integral_constant<int, 1>{});
+  float g[kEdges][4];
+#pragma unroll
+  for (int i = 0; i < kEdges; ++i) g[i][0] = g[i][1] = g[i][2] = g[i][3] = 0.0f;
+  const float* const s = A.s.data + (b0 + kWidth * part);
+  // Where lanes of different column counts share rows, they load four floats all the
+  // same, in one instruction, the ones past the batch being the next neuron's and
+  // left unused; only a row at the plane's very end is loaded column by column.
+  const int64_t end = kWhole || kShare<BT> == 1
+                          ? 0 : (A.N - 1) * A.s.sn + A.B - (b0 + kWidth * part) - kWidth;
+  if (kWhole || (kShare<BT> == 1 && cols >= kWidth)) {
+    gather_columns<BT, kWidth>(s, A.s.sn, c, first, e0, e1, g);
+  } else if (kShare<BT> == 1) {
+    if (cols == 3) gather_columns<BT, 3>(s, A.s.sn, c, first, e0, e1, g);
+    else if (cols == 2) gather_columns<BT, 2>(s, A.s.sn, c, first, e0, e1, g);
+    else if (cols == 1) gather_columns<BT, 1>(s, A.s.sn, c, first, e0, e1, g);
+  } else if (cols > 0) {
+#pragma unroll
+    for (int i = 0; i < kEdges; ++i) {
+      const int64_t at = c[i] * A.s.sn;
+      if (first + i < e0 || first + i >= e1) continue;
+      if (at <= end) {
+        load_columns<kWidth>(s + at, g[i]);
+      } else {
+        for (int k = 0; k < cols; ++k) g[i][k] = s[at + k];
+      }
+    }
+  }
+  if (first >= e1) return;
+#pragma unroll
+  for (int t = 0; t < kWidth; ++t) {
+    if (!kWhole && t >= cols) break;   // nobody reads a column past the batch
+    float* const at = prod + (kWidth * part + t) * kProductStride<BT>;
+#pragma unroll
+    for (int k = 0; k < kShare<BT>; ++k) {
+      v4f pv;
+      pv.x = w[4 * k] * g[4 * k][t];
+      pv.y = w[4 * k + 1] * g[4 * k + 1][t];
+      pv.z = w[4 * k + 2] * g[4 * k + 2][t];
+      pv.w = w[4 * k + 3] * g[4 * k + 3][t];
+      *reinterpret_cast<v4f*>(at + 4 * k) = pv;
+    }
+  }
+}
+
 template <int BT, int FMT>
 __global__ __launch_bounds__(kThreads) void tick_kernel(TickArgs A) {
   constexpr int kPasses = TileCfg<BT>::passes;
   constexpr int kCap = block_capacity<BT>();
-  constexpr int kStride = kCap + 4;  // padded [column][edge] rows keep 16-byte alignment
+  constexpr int kStride = kProductStride<BT>;
   __shared__ __attribute__((aligned(16))) float prod[BT * kStride];
   __shared__ int32_t srow[kMaxRows + 1];
 
@@ -235,56 +350,26 @@ __global__ __launch_bounds__(kThreads) void tick_kernel(TickArgs A) {
   for (int r = tid; r <= nrows; r += kThreads) srow[r] = A.rowptr[r0 + r];
 
   // Phase 1: decode, gather, multiply, stage in LDS.
-  bool paired = false;
-  if constexpr (BT == 8 && kPasses == 1) {
-    // Eight columns of neuron-major s: an edge's source row is 32 bytes.  The
-    // two lanes of a pair take the pair's eight edges together, each loading one
-    // 16-byte half of every edge's row, so one load instruction reads 32 rows
-    // whole and the L2 sees one request per row rather than up to two (the
-    // lanes trade column indices and weights with shuffles).  The products and
-    // their LDS places are those of the per-lane path below, so the sums are
-    // bitwise the same.  N=50k, M=1M, B=8: 14.8 to 13.7 us per tick.
-    if (A.s_vec4 && b0 + 8 <= A.B) {
-      paired = true;
-      const bool have = base + tid * 4 < e1;
-      int c_own[4], c_par[4];
-      float w_own[4], w_par[4];
+  bool staged = false;
+  if constexpr (BT >= 2) {
+    if (A.s_rows) {
+      staged = true;
+      const bool whole = b0 + BT <= A.B;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        c_own[k] = have ? cq[0][k] : 0;
-        w_own[k] = have ? wq[0][k] : 0.0f;
-        c_par[k] = __shfl_xor(c_own[k], 1, 64);
-        w_par[k] = __shfl_xor(w_own[k], 1, 64);
-      }
-      const int h = tid & 1;                         // the half of the row this lane loads
-      const int pair0 = base + (tid & ~1) * 4;       // the pair's first edge
-      v4f g[8];
-      float w[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        // Edges 0-3 are the even lane's quad, 4-7 the odd lane's.
-        const int e = pair0 + i;
-        const int c = i < 4 ? (h ? c_par[i] : c_own[i]) : (h ? c_own[i - 4] : c_par[i - 4]);
-        w[i] = i < 4 ? (h ? w_par[i] : w_own[i]) : (h ? w_own[i - 4] : w_par[i - 4]);
-        g[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        if (e >= e0 && e < e1)
-          g[i] = *reinterpret_cast<const v4f*>(A.s.data + static_cast<int64_t>(c) * A.s.sn +
-                                               (b0 + 4 * h));
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        v4f lo, hi;
-        lo.x = w[0] * g[0][t]; lo.y = w[1] * g[1][t]; lo.z = w[2] * g[2][t]; lo.w = w[3] * g[3][t];
-        hi.x = w[4] * g[4][t]; hi.y = w[5] * g[5][t]; hi.z = w[6] * g[6][t]; hi.w = w[7] * g[7][t];
-        float* const at = prod + (4 * h + t) * kStride + (pair0 - base);
-        *reinterpret_cast<v4f*>(at) = lo;
-        *reinterpret_cast<v4f*>(at + 4) = hi;
+      for (int p = 0; p < kPasses; ++p) {
+        const int q = base + (p * kThreads + tid) * 4;
+        const bool have = q < e1;
+        const int first = base + (p * kThreads + (tid & ~(kShare<BT> - 1))) * 4;
+        if (whole)
+          gather_rows<BT, true>(A, cq[p], wq[p], have, first, e0, e1, b0, prod + (first - base));
+        else
+          gather_rows<BT, false>(A, cq[p], wq[p], have, first, e0, e1, b0, prod + (first - base));
       }
     }
   }
 #pragma unroll
   for (int p = 0; p < kPasses; ++p) {
-    if (paired) break;
+    if (staged) break;
     const int q = base + (p * kThreads + tid) * 4;
     if (q < e1) {
       float g[4][BT];
@@ -293,18 +378,6 @@ __global__ __launch_bounds__(kThreads) void tick_kernel(TickArgs A) {
         const int e = q + k;
         const bool valid = e >= e0 && e < e1;
         const int64_t c = cq[p][k];
-        if constexpr (BT >= 4) {
-          if (A.s_vec4) {
-#pragma unroll
-            for (int j = 0; j < BT; j += 4) {
-              v4f sv = {0.0f, 0.0f, 0.0f, 0.0f};
-              if (valid && b0 + j < A.B)
-                sv = *reinterpret_cast<const v4f*>(A.s.data + c * A.s.sn + (b0 + j));
-              g[k][j] = sv.x; g[k][j + 1] = sv.y; g[k][j + 2] = sv.z; g[k][j + 3] = sv.w;
-            }
-            continue;
-          }
-        }
 #pragma unroll
         for (int j = 0; j < BT; ++j)
           g[k][j] = (valid && b0 + j < A.B) ? A.s.data[(b0 + j) * A.s.sb + c * A.s.sn] : 0.0f;
@@ -369,8 +442,11 @@ int column_tile(int64_t batch) {
   if (batch <= 1) return 1;
   if (batch <= 2) return 2;
   if (batch <= 4) return 4;
-  if (batch <= 8) return 8;
-  return 16;
+  // Wider batches run in tiles of 8 columns: a 16-column tile needs 67 KB of LDS and
+  // 200 registers per lane, two workgroups per compute unit (us per tick at 16 / 8
+  // columns per tile, N=50k, M=1M: B=12 25.4 / 23.2, B=16 27.0 / 25.7, B=24 50.3 /
+  // 40.4; N=30k, M=3M, B=12 48.1 / 44.5).
+  return 8;
 }
 
 int32_t capacity_for(int64_t batch) {
@@ -378,8 +454,7 @@ int32_t capacity_for(int64_t batch) {
     case 1: return block_capacity<1>();
     case 2: return block_capacity<2>();
     case 4: return block_capacity<4>();
-    case 8: return block_capacity<8>();
-    default: return block_capacity<16>();
+    default: return block_capacity<8>();
   }
 }
 
@@ -402,8 +477,7 @@ hipError_t launch_tick(const TickArgs& A, int fmt, hipStream_t stream) {
     case 1: return launch_tile<1>(A, fmt, stream);
     case 2: return launch_tile<2>(A, fmt, stream);
     case 4: return launch_tile<4>(A, fmt, stream);
-    case 8: return launch_tile<8>(A, fmt, stream);
-    default: return launch_tile<16>(A, fmt, stream);
+    default: return launch_tile<8>(A, fmt, stream);
   }
 }
 
@@ -461,12 +535,10 @@ int32_t quad_aligned(const ns_csr& m) {
   return (col % 16 == 0) && (w % need == 0);
 }
 
-int32_t neuron_major_vec4(const ns_plane& s, int64_t batch) {
-  if (column_tile(batch) < 4) return 0;
-  // Exactly neuron-major ([N][B] contiguous, B % 4 == 0): every 4-column group
-  // starting below B lies inside the neuron's row.
-  return s.stride_b == 1 && s.stride_n == batch && batch % 4 == 0 &&
-         reinterpret_cast<uintptr_t>(s.data) % 16 == 0;
+// Whether a source's columns are neighbours in memory (every tensor plane's
+// address is a multiple of 4).
+int32_t neuron_major(const ns_plane& s, int64_t batch) {
+  return batch >= 2 && s.stride_b == 1 && reinterpret_cast<uintptr_t>(s.data) % 4 == 0;
 }
 
 }  // namespace ns
@@ -538,7 +610,7 @@ extern "C" int ns_dendritic_step(const ns_step_args* args, void* stream) {
   A.os = out_plane(a.out_state); A.od = out_plane(a.out_dendrite);
   A.oa = out_plane(a.out_adaptation); A.oj = out_plane(a.out_current);
   A.quad_loads = quad_aligned(a.matrix);
-  A.s_vec4 = neuron_major_vec4(a.state, a.batch);
+  A.s_rows = neuron_major(a.state, a.batch);
   A.spmm_only = 0;
   const hipError_t err = launch_tick(A, a.matrix.format, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail_launch("dendritic tick", err);
@@ -583,7 +655,7 @@ extern "C" int ns_csr_spmm(const ns_spmm_args* args, void* stream) {
   A.bounds = a.plan.bounds; A.n_blocks = a.plan.n_blocks;
   A.os = out_plane(a.out);
   A.quad_loads = quad_aligned(a.matrix);
-  A.s_vec4 = neuron_major_vec4(a.source, a.batch);
+  A.s_rows = neuron_major(a.source, a.batch);
   A.spmm_only = 1;
   A.spmm_accumulate = a.accumulate != 0;
   const hipError_t err = launch_tick(A, a.matrix.format, static_cast<hipStream_t>(stream));

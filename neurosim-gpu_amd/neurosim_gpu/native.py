@@ -1210,7 +1210,7 @@ def plan_rollout(rowptr: np.ndarray, bounds: np.ndarray, batch: int):
     n = rowptr.size - 1
     if not 0 < n <= ROLLOUT_MAX_NEURONS:
         return None
-    tile = 1 if batch <= 1 else 2 if batch <= 2 else 4 if batch <= 4 else 8 if batch <= 8 else 16
+    tile = 1 if batch <= 1 else 2 if batch <= 2 else 4 if batch <= 4 else 8
     capacity = int(load_library().ns_block_edges(int(batch)))
     first_row, first_edge = bounds[:, 0].astype(np.int64), bounds[:, 1].astype(np.int64)
     counts = np.diff(first_row)

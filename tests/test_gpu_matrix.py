@@ -401,3 +401,32 @@ def test_row_blocks_at_every_column_tile(gpu, batch, fmt):
             assert torch.equal(getattr(neuron_major, f), getattr(row_major, f)), (batch, fmt, t, f)
     assert neuron_major.state.stride(0) == 1 or batch == 1
     assert errors(neuron_major, oracle) <= 1e-5
+
+
+@pytest.mark.parametrize("batch", [2, 3, 5, 6, 7, 8, 9, 11, 12, 16, 21])
+@pytest.mark.parametrize("n,m", [(1, 1), (37, 900), (700, 40_000)])
+def test_neuron_major_gathers_at_every_batch(gpu, batch, n, m):
+    """The row-block tick loads a neuron-major state's columns four at a time at any
+    alignment, two lanes per row from five columns on (the last neuron's row column by
+    column): bitwise the tick on the same state stored row-major, which gathers each
+    column by itself, on a state that ends where its allocation ends."""
+    print(f"case row gathers batch={batch} n={n} m={m}", flush=True)
+    case = make_case(n, m, 6, gpu)
+    gen = torch.Generator().manual_seed(batch)
+    planes = [torch.rand(batch, n, generator=gen).to(gpu) for _ in range(3)]
+    drive = column_drive(batch).to(gpu)
+    runs = []
+    for neuron_major in (False, True):
+        native = NativeDendriticMatrixRuntime(case.topology, case.model, planes[0].clone(),
+                                              kernel="rows")
+        state, dendrite, adaptation = (
+            p.t().contiguous().t() if neuron_major else p.clone() for p in planes)
+        native.state, native.dendritic_state, native.adaptation_state = state, dendrite, adaptation
+        native.step(drive, dendritic_drive=0.1)
+        runs.append((native.state, native.dendritic_state, native.adaptation_state))
+    oracle = ort.MatrixOracle(case.graph, case.params, planes[0].cpu())
+    oracle.dendritic_state, oracle.adaptation_state = planes[1].cpu(), planes[2].cpu()
+    oracle.step(drive.cpu(), 0.1)
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
+    assert max_err(runs[1][0], oracle.state) <= 1e-5
