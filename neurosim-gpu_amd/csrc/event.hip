@@ -352,7 +352,12 @@ __global__ __launch_bounds__(kThreads) void event_tick_kernel(EventArgs A) {
 // emitting pairs' bitmap is staged in LDS first, and an edge whose source is
 // silent costs its column index and one LDS read: a stream of 4 bytes per edge
 // with gathers for the active ones only, where the unpruned product is bound by
-// one L2 request per edge.
+// one L2 request per edge.  us per advance and product, 15% of the neurons
+// emitting, at 4 / 8 edges per lane in flight (the lanes per row halved to match):
+// N=166k, B=1 M=10M 29.7 / 29.0, M=25M 63.6 / 48.3; N=50k M=4M B=1 15.6 / 13.4; N=60k
+// M=3M B=16 48.8 / 44.1 (the backward's kernels lose: weight gradient at N=50k,
+// M=4M, B=16 26 / 35).
+constexpr int kProductUnroll = 8;
 constexpr int kProductThreads = 512;
 constexpr int kProductBlocks = 1024;
 constexpr int64_t kProductBitBytes = 64 * 1024;  // largest bitmap staged
@@ -376,25 +381,42 @@ __global__ __launch_bounds__(kProductThreads) void event_product_kernel(EventArg
   const int lane = static_cast<int>(t & (group - 1));
   const int q = lane & (LPE - 1), el = lane / LPE;
   const int64_t B = A.B;
-  for (int64_t n = t >> group_log2; n < A.N; n += step) {
-    const int32_t e0 = A.in_rowptr[n], e1 = A.in_rowptr[n + 1];
+  // A row's bounds load while the row before is summed, and its current before its
+  // edges, so that a row waits for its indices and its gathers only.
+  int64_t n = t >> group_log2;
+  int32_t e0 = 0, e1 = 0;
+  if (n < A.N) {
+    e0 = A.in_rowptr[n];
+    e1 = A.in_rowptr[n + 1];
+  }
+  while (n < A.N) {
+    const int64_t next = n + step;
+    int32_t next0 = 0, next1 = 0;
+    if (next < A.N) {
+      next0 = A.in_rowptr[next];
+      next1 = A.in_rowptr[next + 1];
+    }
     for (int64_t b0 = 0; b0 < B; b0 += kCols) {
       const int64_t b = b0 + q * VL;
       const bool have = b < B;
+      float* const at0 = A.current + (have ? b : 0) * A.csb + n * A.csn;
+      float before[VL];
+#pragma unroll
+      for (int k = 0; k < VL; ++k) before[k] = el == 0 ? at0[(have ? k : 0) * A.csb] : 0.0f;
       float acc[VL];
 #pragma unroll
       for (int k = 0; k < VL; ++k) acc[k] = 0.0f;
-      for (int32_t e = e0 + el; e < e1; e += edge_lanes * kEdgeUnroll) {
-        int32_t c[kEdgeUnroll];
-        float w[kEdgeUnroll], x[kEdgeUnroll][VL];
+      for (int32_t e = e0 + el; e < e1; e += edge_lanes * kProductUnroll) {
+        int32_t c[kProductUnroll];
+        float w[kProductUnroll], x[kProductUnroll][VL];
 #pragma unroll
-        for (int u = 0; u < kEdgeUnroll; ++u) {
+        for (int u = 0; u < kProductUnroll; ++u) {
           const int32_t at = min(e + edge_lanes * u, e1 - 1);
           c[u] = A.in_col[at];
           if constexpr (!kBits) w[u] = A.weight[at];
         }
 #pragma unroll
-        for (int u = 0; u < kEdgeUnroll; ++u) {
+        for (int u = 0; u < kProductUnroll; ++u) {
           const int32_t at = e + edge_lanes * u;
           if constexpr (kBits) {
             // Batch 1 or 2: the source's bits lie in one word, at c * B.
@@ -414,7 +436,7 @@ __global__ __launch_bounds__(kProductThreads) void event_product_kernel(EventArg
           }
         }
 #pragma unroll
-        for (int u = 0; u < kEdgeUnroll; ++u) {
+        for (int u = 0; u < kProductUnroll; ++u) {
 #pragma unroll
           for (int k = 0; k < VL; ++k)
             acc[k] = x[u][k] != 0.0f ? __builtin_fmaf(w[u], x[u][k], acc[k]) : acc[k];
@@ -426,12 +448,12 @@ __global__ __launch_bounds__(kProductThreads) void event_product_kernel(EventArg
       }
       if (el == 0 && have) {
 #pragma unroll
-        for (int k = 0; k < VL; ++k) {
-          float* const at = A.current + (b + k) * A.csb + n * A.csn;
-          *at = *at + acc[k];
-        }
+        for (int k = 0; k < VL; ++k) at0[k * A.csb] = before[k] + acc[k];
       }
     }
+    n = next;
+    e0 = next0;
+    e1 = next1;
   }
 }
 
@@ -441,7 +463,7 @@ hipError_t launch_product(const EventArgs& A, int64_t n_edges, hipStream_t s) {
   const bool pruned = A.emitting && bit_bytes <= kProductBitBytes &&
                       (A.B == 1 || (A.B == 2 && aligned));
   const EdgeForm form = edge_form(A.B, aligned);
-  const int lg = edge_lanes_for(n_edges, A.N, form.lpe);
+  const int lg = edge_lanes_for(n_edges, A.N, form.lpe, kProductUnroll);
   const int64_t lanes = A.N * (form.lpe << lg);
   const dim3 grid(static_cast<unsigned>(
       std::min<int64_t>((lanes + kProductThreads - 1) / kProductThreads,

@@ -361,7 +361,7 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
       if (int rc = panel_step(transposed, s, 2, true)) return rc;
     } else if (want_state) {
       const EdgeForm form = edge_form(batch, gj_rows);
-      const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe);
+      const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe, kEdgeUnroll);
       with_edge_form(form, [&](auto vl, auto lpe) {
         transposed_product_kernel<vl(), lpe()><<<lanes_grid(n, form.lpe << lg), kGradThreads, 0, s>>>(
             a.out_rowptr, a.dst, a.out_weight_index, static_cast<const float*>(a.matrix.weight),
@@ -383,7 +383,7 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
                          reinterpret_cast<uintptr_t>(from.data) % (4 * width) == 0 &&
                          reinterpret_cast<uintptr_t>(g) % (4 * width) == 0;
       const EdgeForm form = edge_form(cols, whole);
-      const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe);
+      const int lg = edge_lanes_for(a.matrix.n_edges, n, form.lpe, kEdgeUnroll);
       with_edge_form(form, [&](auto vl, auto lpe) {
         weight_gradient_kernel<vl(), lpe()><<<lanes_grid(n, form.lpe << lg), kGradThreads, 0, s>>>(
             a.matrix.rowptr, a.matrix.col, g, from, n, cols, a.d_weight,

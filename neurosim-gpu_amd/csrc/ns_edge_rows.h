@@ -9,14 +9,14 @@
 
 namespace ns {
 
-constexpr int kEdgeUnroll = 4;  // edges per lane per round of the edge loops
+constexpr int kEdgeUnroll = 4;  // edges per lane per round of the backward's edge loops
 
 // The edge kernels of the backward and of the event tick give each row (a source,
-// or a destination) a power-of-two group of lanes: LPE lanes per edge, VL neighbouring columns each
-// (one 4 * VL byte load of a neuron-major row; VL = 1 takes any strides), and
-// `edge_lanes` edges at a time, kEdgeUnroll rounds of them in flight.  The host
-// picks edge_lanes so that a row of average length is about one round
-// (edge_lanes_for).  A wavefront per row, every lane walking its edge's columns
+// or a destination) a power-of-two group of lanes: LPE lanes per edge, VL
+// neighbouring columns each (one 4 * VL byte load of a neuron-major row; VL = 1
+// takes any strides), and `edge_lanes` edges at a time, `unroll` rounds of them in
+// flight.  The host picks edge_lanes so that a row of average length is about
+// one round (edge_lanes_for).  A wavefront per row, every lane walking its edge's columns
 // by itself, left two thirds of the lanes idle at 20 edges per row and read
 // each gathered row in 4-byte pieces.
 
@@ -33,11 +33,11 @@ __device__ __forceinline__ void load_row(const float* at, float x[VL]) {
 }
 
 // log2 of the edges a row's group takes at a time: the smallest power of two for
-// which kEdgeUnroll of them cover a row of average length, at most what fits
+// which `unroll` of them cover a row of average length, at most what fits
 // one wavefront beside the LPE lanes of an edge.
-inline int edge_lanes_for(int64_t edges, int64_t rows, int lpe) {
+inline int edge_lanes_for(int64_t edges, int64_t rows, int lpe, int unroll) {
   int lg = 0;
-  while ((lpe << lg) < 64 && (int64_t{kEdgeUnroll} << lg) * rows < edges) ++lg;
+  while ((lpe << lg) < 64 && (int64_t{unroll} << lg) * rows < edges) ++lg;
   return lg;
 }
 

@@ -734,8 +734,8 @@ def product_break_even(n_edges: int, batch: int) -> float:
     Crossings measured (N, M, B, thousands of active out-edges): 50k 4M 1, 180;
     166k 10M 1, 380; 300k 15M 1, 610; 166k 25M 1, 960; 50k 2M 3, 310; 100k 4M 5,
     1030; and where the scatter adds runs of columns, 60k 5M 2, 180; 60k 3M 4,
-    370; 50k 1M 8, 260; 60k 3M 16, 1070.  At 12% activity, us per tick, scatter /
-    product: 166k 10M 1, 68 / 29; 166k 25M 1, 164 / 62; 50k 1M 8, 41 / 19."""
+    370; 50k 1M 8, 260; 60k 3M 16, 1070.  At 12% activity, us per eager tick, scatter
+    / product: 166k 10M 1, 68 / 29; 166k 25M 1, 164 / 48; 50k 1M 8, 41 / 19."""
     runs = 2 <= batch <= 64 and batch & (batch - 1) == 0
     return 100_000 + (0.02 if runs else 0.034) * n_edges * batch
 
