@@ -721,23 +721,27 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
 
 
 # Fewest edges times columns for which the scatter's tick may become an advance and
-# an in-edge product (NS_EVENT_PRODUCT).  Below, an eager tick is bound by its host
-# side, which a second launch makes longer (N=50k, M=1M, B=1: 12.7 us per scattered
-# tick at 12% activity, 19.6 with the product).
-PRODUCT_MIN_EDGES = 4_000_000
+# an in-edge product (NS_EVENT_PRODUCT).  Below, the product's second launch (an eager
+# tick of 14.5 us, host-bound) pays only when more than a tenth of the edges is
+# active, and the counts cost half a microsecond per tick.
+PRODUCT_MIN_EDGES = 1_500_000
 
 
 def product_break_even(n_edges: int, batch: int) -> float:
     """Active out-edges of a tick from which the in-edge product beats the scatter.
 
-    The scatter's cost is its atomics, the product's the stream of the edges.
-    Crossings measured (N, M, B, thousands of active out-edges): 50k 4M 1, 180;
-    166k 10M 1, 380; 300k 15M 1, 610; 166k 25M 1, 960; 50k 2M 3, 310; 100k 4M 5,
-    1030; and where the scatter adds runs of columns, 60k 5M 2, 180; 60k 3M 4,
-    370; 50k 1M 8, 260; 60k 3M 16, 1070.  At 12% activity, us per eager tick, scatter
-    / product: 166k 10M 1, 68 / 29; 166k 25M 1, 164 / 48; 50k 1M 8, 41 / 19."""
-    runs = 2 <= batch <= 64 and batch & (batch - 1) == 0
-    return 100_000 + (0.02 if runs else 0.034) * n_edges * batch
+    The scatter's cost is its atomics, the product's the stream of the edges, and
+    the host side of its second launch on small graphs.  Crossings measured (N, M, B,
+    thousands of active out-edges): 50k 1.5M 1, 150; 30k 2M 1, 120; 13k 1.2M 3, 110;
+    50k 4M 1, 130; 166k 10M 1, 440; 300k 15M 1, 560; 166k 25M 1, 760; 100k 4M 5, 1000;
+    and where the scatter adds runs of columns, 60k 5M 2, 190; 60k 3M 4, 350; 50k 1M 8,
+    240; 60k 3M 16, 800.  At 12-15% activity, us per eager tick, scatter / product:
+    166k 10M 1, 68 / 29; 166k 25M 1, 164 / 48; 30k 2M 1, 27 / 15; 13k 1.2M 3, 40 /
+    15; 50k 1M 8, 41 / 18."""
+    slots = n_edges * batch
+    if 2 <= batch <= 64 and batch & (batch - 1) == 0:
+        return max(200_000, 100_000 + 0.02 * slots)
+    return max(150_000, 60_000 + 0.03 * slots)
 
 
 class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
@@ -886,6 +890,8 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
         """Apply a finished sample and say whether this tick samples (counts its
         active out-edges).  "auto" does so at policy ticks; the scatter of a large
         graph (``_adaptive``) applies a sample on the first tick that finds it done."""
+        if self._activity is None:
+            return False
         phase = self._tick % self.policy_interval
         if self._adaptive:
             due = phase == self.policy_interval // 2     # past the start state's transient
@@ -893,7 +899,7 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
                 return False
         else:
             due = phase == 0
-            if self.propagation != "auto" or not due:
+            if not due:
                 return False
         if torch.cuda.is_current_stream_capturing():
             return False
