@@ -241,24 +241,33 @@ class _Recording:
     ticks adds no pair of gradients outside the kernels (seven torch additions per
     tick otherwise).  The gradient of the third, when there is one, is the entry of
     the tick after, whose weight gradient this tick's pass over the edges computes
-    together with its own.  The states are held weakly:
-    once the caller drops them the tokens, and the graph behind them, go too."""
+    together with its own.  One tick at most takes the tokens: autograd would add
+    what two takers return for them, and pending entries cannot be added.  A second
+    one (a shallow copy of the runtime, or one rewound to saved attributes) starts a
+    run of its own.  The states are held weakly: once the caller drops them the
+    tokens, and the graph behind them, go too."""
 
-    __slots__ = ("states", "weight", "params", "versions", "topology", "stream", "tokens")
+    __slots__ = ("states", "weight", "params", "versions", "topology", "stream", "_tokens")
 
     def __init__(self, states, weight, params, versions, topology, stream, tokens) -> None:
         self.weight, self.params, self.topology, self.stream = weight, params, topology, stream
-        self.versions, self.tokens = versions, tokens
-        self.states = (weakref.ref(states[0], self._drop), *map(weakref.ref, states[1:]))
+        self.versions = versions
+        self._tokens = held = [tokens]
+        self.states = (weakref.ref(states[0], lambda _: held.clear()),
+                       *map(weakref.ref, states[1:]))
 
-    def _drop(self, _) -> None:
-        self.tokens = None
-
-    def continues(self, states, weight, params, versions, topology, stream) -> bool:
-        return (self.tokens is not None and topology is self.topology
+    def take(self, states, weight, params, versions, topology, stream) -> tuple | None:
+        """The tokens, if a tick on these inputs continues the run and is the first to;
+        else None."""
+        if not (topology is self.topology
                 and all(ref() is s for ref, s in zip(self.states, states))
                 and weight is self.weight and all(map(is_, params, self.params))
-                and stream == self.stream and versions == self.versions)
+                and stream == self.stream and versions == self.versions):
+            return None
+        try:
+            return self._tokens.pop()
+        except IndexError:
+            return None
 
 
 class _NativeTick(torch.autograd.Function):
@@ -704,14 +713,15 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
         stream = current_stream(self.state.device)
         recording = self._recording
         versions = [(t._version, t.requires_grad) for t in (weight, *params)]
-        first = recording is None or not recording.continues(states, weight, params, versions,
-                                                             topology, stream)
+        linked = (recording.take(states, weight, params, versions, topology, stream)
+                  if recording is not None else None)
+        first = linked is None
         info = _TickInfo(extension=self.extension, topology=topology, us=us, vs=vs, tick=tick,
                          source_major=self.source_major_weights, transposed=transposed,
                          prepared=self._prepared_backward, by_neuron=by_neuron, weight=weight,
                          params=params, first=first)
-        linked = (weight, *params) if first else recording.tokens
-        s, d, a, *tokens = _NativeTick.apply(info, *states, u, v, *linked)
+        s, d, a, *tokens = _NativeTick.apply(info, *states, u, v,
+                                             *((weight, *params) if first else linked))
         states = (s, d, a)
         self._recording = _Recording(states, weight, params, versions, topology, stream,
                                      tuple(tokens))

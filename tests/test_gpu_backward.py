@@ -17,6 +17,8 @@ from the second backward of a weight version on.
 
 from __future__ import annotations
 
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -450,6 +452,48 @@ def test_a_run_of_recorded_ticks_ends_where_its_inputs_change(gpu):
     for a, b in zip(gradients(True), gradients(False)):
         # branches meet in another order of additions: a few roundings of the sum
         assert float((a - b).abs().max()) <= 2.0 ** -20 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("batch,kernel", [(1, "panels"), (3, "rows")])
+@pytest.mark.parametrize("how", ["copy", "rewind"])
+def test_a_run_is_continued_once(gpu, batch, kernel, how):
+    """A simulation branched by a shallow copy of its runtime, or rewound to saved
+    attributes: both branches start from the same recorded states, and only one may
+    continue that run.  Gradients match those of ticks recorded one by one."""
+    print(f"case backward branches batch={batch} kernel={kernel} {how}", flush=True)
+    g = graph(500, 6_000, 6)
+    inputs = inputs_for(g, batch, 21)
+
+    def gradients(linked: bool):
+        topo = topology(g, torch.float32, gpu)
+        topo.in_weight.requires_grad_(True)
+        mdl = model(inputs["params"], torch.float32, gpu, False)
+        rt = NativeDendriticMatrixRuntime(topo, mdl, torch.full((batch, 500), .3, device=gpu),
+                                          kernel=kernel)
+
+        def step(runtime, u):
+            runtime.step(u, dendritic_drive=0.1)
+            if not linked:
+                runtime._recording = None
+
+        for u in (0.1, 0.2):
+            step(rt, u)
+        other = copy.copy(rt)
+        kept = dict(vars(rt))
+        step(rt, 0.5)              # odd numbers of ticks: both branches leave an entry pending
+        loss = (rt.state ** 2).sum()
+        if how == "rewind":
+            vars(rt).update(kept)
+            other = rt
+        for u in (0.1, 0.4, 0.2):
+            step(other, u)
+        loss = loss + (other.state * 0.7).sum()
+        return torch.autograd.grad(loss, [topo.in_weight, *params_of(mdl)])
+
+    for a, b in zip(gradients(True), gradients(False)):
+        # Five ticks of at most three columns meet in another order: 15 additions of
+        # partial sums below twice the largest gradient.
+        assert float((a - b).abs().max()) <= 2.0 ** -19 * float(b.abs().max())
 
 
 @pytest.mark.parametrize("n,m,chunk,bucket", [
