@@ -414,7 +414,8 @@ typedef struct ns_step_grad_args {
   float* pending;              /* optional float32[2][N][2*B]: what the weight gradients of two
                                   ticks are made of, the gradients of j (first N*2B floats) and
                                   the states, entry e of neuron n in columns e*B to e*B + B.
-                                  This tick's are stored as entry `pending_entry`, and the
+                                  This tick's are stored as entry `pending_entry` (entry 0
+                                  also zeroes entry 1, so the block is whole), and the
                                   weight gradient is left to the call that stores entry 1: it
                                   gives d_weight both ticks' in one pass over the edges
                                   (`d_weight` must be NULL with entry 0). */

@@ -42,6 +42,7 @@ struct GradArgs {
   float* gp[6];
   int32_t add_params;    // add to gp instead of storing
   OutPlane pg, ps;       // optional copies of gj and s (the pending entry)
+  int64_t clear;         // floats from the entry to the one to zero (0: none)
 };
 
 // One lane per (neuron, column), LB lanes per neuron; lane q takes columns q,
@@ -96,6 +97,10 @@ __global__ __launch_bounds__(kGradThreads) void advance_backward_kernel(GradArgs
     if (A.pg.data) {
       A.pg.put(b, n, g_j);
       A.ps.put(b, n, s);
+      if (A.clear) {
+        A.pg.put(b + A.clear, n, 0.0f);
+        A.ps.put(b + A.clear, n, 0.0f);
+      }
     }
   }
   float sums[6] = {g_alpha, g_gain, g_rho_d, g_rho_a, g_c, g_k};
@@ -321,6 +326,7 @@ extern "C" int ns_dendritic_step_backward(const ns_step_grad_args* args, void* s
     float* const entry = a.pending + a.pending_entry * batch;
     G.pg = OutPlane{entry, 1, 2 * batch};
     G.ps = OutPlane{entry + 2 * batch * n, 1, 2 * batch};
+    G.clear = a.pending_entry == 0 ? batch : 0;
   }
   // The transposed product on panels: W^T @ gj added into d_state.
   ns_step_args transposed{};

@@ -1504,9 +1504,9 @@ class PreparedBackward:
     weight gradient and the parameter gradients' block of later ticks, which this
     tick's are added to in place (as autograd would add them, in the same order).
     ``pending`` ([2, N, 2B]) defers the weight gradient: a call with
-    ``pending_entry`` 0 only stores what its own is made of, the next one, with 1, gives
-    both ticks' in one pass.  Last of the results is the parameter gradients' block; ``split=False`` leaves
-    out the list of its rows."""
+    ``pending_entry`` 0 only stores what its own is made of (and zeroes entry 1), the
+    next one, with 1, gives both ticks' in one pass.  Last of the results is the
+    parameter gradients' block; ``split=False`` leaves out the list of its rows."""
 
     def __init__(self, extension: "NativeExtension", state: torch.Tensor, params, rowptr, col,
                  weight, out_rowptr, dst, weight_index):

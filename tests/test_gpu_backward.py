@@ -496,6 +496,44 @@ def test_a_run_is_continued_once(gpu, batch, kernel, how):
         assert float((a - b).abs().max()) <= 2.0 ** -19 * float(b.abs().max())
 
 
+@pytest.mark.parametrize("ticks", [2, 3])
+@pytest.mark.parametrize("batch,kernel", [(1, "panels"), (3, "rows")])
+def test_recorded_ticks_pass_anomaly_detection(gpu, batch, kernel, ticks):
+    """No gradient that a tick hands on holds memory it has not written: with new memory
+    filled with NaN, a backward under anomaly detection (which refuses NaN in any
+    gradient, those between the ticks among them) passes and gives the gradients of
+    ticks recorded one by one."""
+    print(f"case backward anomaly batch={batch} kernel={kernel} ticks={ticks}", flush=True)
+    g = graph(500, 6_000, 3)
+    inputs = inputs_for(g, batch, 33)
+
+    def gradients(linked: bool):
+        topo = topology(g, torch.float32, gpu)
+        topo.in_weight.requires_grad_(True)
+        mdl = model(inputs["params"], torch.float32, gpu, False)
+        rt = NativeDendriticMatrixRuntime(topo, mdl, torch.full((batch, 500), .3, device=gpu),
+                                          kernel=kernel)
+        for t in range(ticks):
+            rt.step(0.1 + 0.1 * t, dendritic_drive=0.1)
+            if not linked:
+                rt._recording = None
+        return torch.autograd.grad(rt.state, [topo.in_weight, *params_of(mdl)],
+                                   grad_outputs=torch.ones_like(rt.state))
+
+    separate = gradients(False)
+    before = torch.are_deterministic_algorithms_enabled()
+    torch.use_deterministic_algorithms(True, warn_only=True)    # fills new memory with NaN
+    try:
+        with torch.autograd.set_detect_anomaly(True):
+            linked = gradients(True)
+    finally:
+        torch.use_deterministic_algorithms(before)
+    for a, b in zip(linked, separate):
+        # 3 ticks' products of at most 3 columns, summed two ticks at a time: nine
+        # additions of partial sums below twice the largest gradient.
+        assert float((a - b).abs().max()) <= 2.0 ** -19 * float(b.abs().max())
+
+
 @pytest.mark.parametrize("n,m,chunk,bucket", [
     (50, 400, None, None), (3000, 90_000, None, None), (3000, 90_000, 4, 64),
     (700, 9_217, 9216, 128), (2000, 60_000, 36_864, 36_864), (300, 5_001, 4_996, 18_432)])
