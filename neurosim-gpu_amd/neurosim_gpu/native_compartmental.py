@@ -207,9 +207,7 @@ class TransposedPanels:
         or ``weight`` gathered into slot order once (see above)."""
         key = self._version(weight)
         self._seen += 1
-        # No copy inside a capture: it would be filled only when the graph replays.
-        late = self.layout.blocked is None and self._seen < 2 and self._expected < 2
-        if late or (self.layout._slot_key != key and torch.cuda.is_current_stream_capturing()):
+        if self.layout.blocked is None and self._seen < 2 and self._expected < 2:
             if self._indexed is None:
                 self._indexed = self.layout.indexed_plan_struct()
             return self._indexed
@@ -307,6 +305,11 @@ class _NativeTick(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_state, grad_dendrite, grad_adaptation, sum_weight, sum_params,
                  pending):
+        # A captured backward has ended the process (a segmentation fault inside the
+        # runtime when the capture ended, cause not known), and it would read copies of
+        # the weights that the replays do not renew.
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("the backward of recorded ticks cannot be captured into a graph")
         info = ctx.info
         topology = info.topology
         saved = list(ctx.saved_tensors)
@@ -520,7 +523,8 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
         training loop through several), the copy is built for the first already
         (N=166k, M=25M, two ticks: copy 65 + 2 x 33 us against indexed 80, copy
         65 and 33).  A version is (tensor, in-place version counter), so an
-        update of the weights is never missed.
+        update of the weights is never missed.  Under graph capture weights that are
+        trained, or seen once, are read in place, so that the replays follow them.
         """
         if self._panels is None:
             return None
@@ -528,6 +532,9 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
         if key != self._recorded_key or self._recorded_source is not weight:
             self._recorded_before = self._recorded_seen
             self._recorded_key, self._recorded_source, self._recorded_seen = key, weight, 0
+        if torch.cuda.is_current_stream_capturing() and (weight.requires_grad
+                                                         or self._recorded_seen < 2):
+            return self._panels.indexed_plan_struct()
         self._recorded_seen += 1
         if self._recorded_seen < 2 and self._recorded_before < 2:
             return self._panels.indexed_plan_struct()

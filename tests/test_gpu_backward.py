@@ -534,6 +534,106 @@ def test_recorded_ticks_pass_anomaly_detection(gpu, batch, kernel, ticks):
         assert float((a - b).abs().max()) <= 2.0 ** -19 * float(b.abs().max())
 
 
+@pytest.mark.skip(reason="capturing a backward ended the process with a segmentation fault in "
+                  "the runtime's end of capture, cause not known; it is refused since")
+@pytest.mark.parametrize("batch,kernel,blocked", [(1, "panels", True), (1, "panels", False),
+                                                  (3, "rows", False)])
+@pytest.mark.parametrize("ticks", [1, 3])
+def test_captured_training_pass_follows_its_weights(gpu, monkeypatch, batch, kernel, blocked,
+                                                    ticks):
+    """A forward and backward captured after one eager pass on the same weight version:
+    replays after in-place updates of the weights give the states and gradients of eager
+    passes on the new weights, the transposed product's among them."""
+    print(f"case backward capture batch={batch} kernel={kernel} blocked={blocked} "
+          f"ticks={ticks}", flush=True)
+    from neurosim_gpu import native_compartmental as nc
+
+    monkeypatch.setattr(nc, "BLOCKED_MIN_EDGES", 0 if blocked else 1 << 60)
+    g = graph(1500, 30_000, 14)
+    inputs = inputs_for(g, batch, 41)
+    probe = torch.tensor(inputs["probe"]["s"], dtype=torch.float32, device=gpu)
+
+    def build(weight):
+        topo = topology(g, torch.float32, gpu)
+        if weight is not None:
+            topo.in_weight.copy_(weight)
+        topo.in_weight.requires_grad_(True)
+        start = [leaf(inputs[k], torch.float32, gpu) for k in ("state", "dendrite", "adaptation")]
+        mdl = model(inputs["params"], torch.float32, gpu, False)
+        rt = NativeDendriticMatrixRuntime(topo, mdl, start[0].detach(), kernel=kernel)
+
+        def one_pass():
+            rt.state, rt.dendritic_state, rt.adaptation_state = start
+            for t in range(ticks):
+                rt.step(0.1 + 0.1 * t, dendritic_drive=0.1)
+            grads = torch.autograd.grad(rt.state, [*start, topo.in_weight, *params_of(mdl)],
+                                        grad_outputs=probe)
+            return (rt.state.detach(), *grads)
+
+        return topo, one_pass
+
+    topo, one_pass = build(None)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        one_pass()
+        captured = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(captured, stream=side):
+            replayed = one_pass()
+    torch.cuda.current_stream().wait_stream(side)
+    for scale in (0.5, -1.5, 1.0):
+        with torch.no_grad():
+            topo.in_weight.mul_(scale)
+        captured.replay()
+        want = build(topo.in_weight.detach())[1]()
+        torch.cuda.synchronize()
+        for a, b in zip(replayed, want):
+            # float32 sums of the same terms, of at most a hundred each
+            assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max())
+
+
+def test_recorded_ticks_under_capture_keep_no_copy_of_trained_weights(gpu, monkeypatch):
+    """What a capture would bake in, without one (the query alone says that the stream is
+    captured): the forward reads trained weights in place, also where a training loop's
+    eager ticks have made a slot-order copy of them, and the backward is refused before
+    it launches anything.  The eager pass after it is right."""
+    print("case backward under capture", flush=True)
+    from neurosim_gpu.native import PANEL_INDEXED
+
+    g = graph(1500, 30_000, 14)
+    inputs = inputs_for(g, 1, 41)
+    topo = topology(g, torch.float32, gpu)
+    topo.in_weight.requires_grad_(True)
+    mdl = model(inputs["params"], torch.float32, gpu, False)
+    start = leaf(inputs["state"], torch.float32, gpu)
+    rt = NativeDendriticMatrixRuntime(topo, mdl, start.detach(), kernel="panels")
+    zero = torch.zeros_like(start)
+
+    def one_pass(ticks):
+        rt.state, rt.dendritic_state, rt.adaptation_state = start, zero, zero
+        for t in range(ticks):
+            rt.step(0.1 + 0.1 * t, dendritic_drive=0.1)
+        return rt.state
+
+    def gradients(out):
+        return torch.autograd.grad(out, [start, topo.in_weight],
+                                   grad_outputs=torch.ones_like(out), retain_graph=True)
+
+    gradients(one_pass(2))
+    with torch.no_grad():
+        topo.in_weight.mul_(0.5)
+    out = one_pass(1)
+    want = gradients(out)
+    with monkeypatch.context() as patched:
+        patched.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        assert rt._recorded_panel_plan(topo.in_weight).flags & PANEL_INDEXED
+        with pytest.raises(RuntimeError, match="cannot be captured"):
+            gradients(out)
+    for a, b in zip(gradients(one_pass(1)), want):
+        # the same terms (panels against row blocks), of at most a hundred each
+        assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max())
+
+
 @pytest.mark.parametrize("n,m,chunk,bucket", [
     (50, 400, None, None), (3000, 90_000, None, None), (3000, 90_000, 4, 64),
     (700, 9_217, 9216, 128), (2000, 60_000, 36_864, 36_864), (300, 5_001, 4_996, 18_432)])
