@@ -592,13 +592,18 @@ class BlockedPermutation:
                  bucket: int | None = None) -> None:
         # us per call (chunk / bucket) on transposed panel layouts: 25M edges 128 at
         # 18432 / 18432, 120 at 18432 / 36864, 220 at 9216 / 9216; 10M 48, 58, 59; 4M
-        # 29, 36, 25; slot by slot (ns_gather_slot_weights) 418, 148 and 57.
+        # 29, 36, 25; slot by slot (ns_gather_slot_weights) 418, 148 and 57.  A run
+        # shortens as the edges grow in number (26 values at 25M, 7 at 100M): 50M 257
+        # at 18432 / 36864 against 768 slot by slot, 100M 546 / 1331, 200M 1498 / 2499.
         half = BLOCKED_MAX // 2
         chunk = chunk or (half if n_edges >= 6_000_000 else half // 2)
         bucket = bucket or (BLOCKED_MAX if n_edges >= 20_000_000 else chunk)
         device, n_slots = perm.device, perm.numel()
         chunks = -(-n_edges // chunk)
         buckets = -(-n_slots // bucket)
+        if chunks * buckets >= 1 << 31:
+            raise RuntimeError(f"a blocked permutation numbers its {chunks} x {buckets} runs in "
+                               "32 bits")
         slots = torch.nonzero(perm >= 0).view(-1).to(torch.int32)
         if slots.numel() != n_edges:
             raise RuntimeError("a blocked permutation holds every edge in one slot")

@@ -151,10 +151,13 @@ class SourceMajorWeights:
         return self._values
 
 
-# Fewest edges for which the transposed weights are permuted in two streaming passes
-# before their first use.  us per product on new weights, indexed / copy + streamed:
-# 4M edges, B=1 37 / 25 + 13; 10M, B=2 107 / 48 + 27; 25M, B=1 334 / 120 + 33.
+# Fewest and most edges for which the transposed weights are permuted in two streaming
+# passes before their first use.  us per product on new weights, indexed / copy + streamed:
+# 4M edges, B=1 37 / 25 + 13; 10M, B=2 107 / 48 + 27; 25M, B=1 334 / 120 + 33.  The
+# passes' runs shorten as the edges grow in number: at 200M, the most measured, the
+# permutation takes 0.6 of the slot gather's time (0.3 at 25M).
 BLOCKED_MIN_EDGES = 4_000_000
+BLOCKED_MAX_EDGES = 200_000_000
 
 
 class TransposedPanels:
@@ -168,8 +171,8 @@ class TransposedPanels:
     The slot-order copy, one random read per edge, is made on the first request
     when ``expect`` has announced two or more products of the version
     (backpropagation through several ticks), else on the second (repeated passes
-    on fixed weights), and streamed after that.  From ``BLOCKED_MIN_EDGES`` edges
-    on the copy is made at once: two streaming passes (``BlockedPermutation``) cost
+    on fixed weights), and streamed after that.  From ``BLOCKED_MIN_EDGES`` to
+    ``BLOCKED_MAX_EDGES`` edges the copy is made at once: two streaming passes (``BlockedPermutation``) cost
     less than the indexed product's reads (N=166k, M=25M: copy 120 us and streamed
     product 33 against 334 indexed; slot by slot the copy took 418).
     Built on the host from the source-major view (set-up only, like the
@@ -184,7 +187,7 @@ class TransposedPanels:
         owi = topology.out_weight_index.to(device=device, dtype=torch.int32)
         self.layout.perm = torch.where(perm >= 0, owi[perm.clamp(min=0).long()],
                                        perm).to(torch.int32).contiguous()
-        if topology.n_edges >= BLOCKED_MIN_EDGES:
+        if BLOCKED_MIN_EDGES <= topology.n_edges <= BLOCKED_MAX_EDGES:
             self.layout.blocked = BlockedPermutation(self.layout.perm, topology.n_edges)
         self._key, self._source, self._seen, self._expected = None, None, 0, 0
         self._indexed = None

@@ -11,6 +11,7 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
 from neurosim_gpu import native
 
@@ -703,3 +704,32 @@ def test_blocked_permutation_validation_messages(lib):
         rc, message = call(**fields)
         assert rc != 0 and text in message, (fields, message)
     assert call(n_slots=0, n_buckets=0)[0] == 0
+
+
+def test_blocked_permutation_is_bounded():
+    """The tables number their runs (chunks times buckets) in 32 bits: more are refused
+    before anything is built, and the sizes that take the permutation stay far below."""
+    from neurosim_gpu import native_compartmental as nc
+
+    edges = 190_000                                # 47500 chunks and buckets of four
+    with pytest.raises(RuntimeError, match="in 32 bits"):
+        native.BlockedPermutation(torch.arange(edges, dtype=torch.int32), edges, 4, 4)
+    most = nc.BLOCKED_MAX_EDGES
+    half = native.BLOCKED_MAX // 2
+    assert nc.BLOCKED_MIN_EDGES < most
+    assert (most // half + 1) * (2 * most // half + 1) < 2 ** 31   # up to twice as many slots
+    # Small tables on the CPU: every edge's value lands in its slot.
+    perm = torch.tensor([3, -1, 0, 4, 1, 2, -1, 5], dtype=torch.int32)
+    place, starts, targets, bucket_start, source = (
+        t.long() for t in native.BlockedPermutation(perm, 6, 4, 4)._tables)
+    work = torch.full((6,), -1)
+    for chunk in range(2):
+        base, count = 4 * chunk, min(4, 6 - 4 * chunk)
+        held = torch.empty(count, dtype=torch.long)
+        held[place[base:base + count]] = torch.arange(base, base + count)
+        for bucket in range(2):
+            a, b = starts[chunk, bucket], starts[chunk, bucket + 1]
+            work[targets[chunk, bucket]:targets[chunk, bucket] + b - a] = held[a:b]
+    slots = [int(work[bucket_start[k // 4] + source[k]]) if source[k] >= 0 else -1
+             for k in range(8)]
+    assert slots == perm.tolist()
