@@ -5,7 +5,7 @@ them: tick i reads set i % 2 and writes set (i+1) % 2, so an even number of
 ticks ends where it started and the captured graph can be replayed back to
 back with no copy, no allocation and no host work per tick.  A network small
 enough for one compute unit per column runs the whole chunk in one launch instead
-(``RolloutLauncher``), in place on the first set.
+(``RolloutLauncher``), in place on the first set; its graph is that one launch.
 
 Inputs can be staged per tick, as in the reference's CUDA-graph rollout of its
 drift benchmark (benchmarks/precision_drift.py:74-143): a drive given as a
@@ -48,9 +48,10 @@ class MatrixRollout:
     weight payload (or its slot-order copy), which the rollout keeps alive, so
     build a new rollout to follow a weight change.  The runtime's current
     states seed the rollout; ``write_back()`` hands the rolled-out states back.
-    ``trace=True`` also copies each tick's new somatic state into ``trace``
-    ([ticks, B, N], overwritten by every replay or ``advance``), one device
-    copy per tick inside the graph.
+    ``trace=True`` also writes each tick's new somatic state into ``trace``
+    ([ticks, B, N], overwritten by every replay or ``advance``): the one-launch
+    rollout writes it itself, the others make one device copy per tick inside
+    the graph.  ``graph`` is the captured chunk (None with ``use_graph=False``).
     """
 
     def __init__(self, runtime, ticks: int, *, drive=0.0, dendritic_drive=0.0,
@@ -96,7 +97,7 @@ class MatrixRollout:
         self._resident = (RolloutLauncher.build(extension, self._launch, topology.in_rowptr, ticks,
                                                 self._sets[0], staged, self.trace)
                           if use_graph else None)
-        if use_graph and self._resident is None:
+        if use_graph:
             self._capture()
 
     def _eager(self, count: int | None = None) -> None:
@@ -111,12 +112,16 @@ class MatrixRollout:
         saved = [p.clone() for p in self._sets[0]]
         side = torch.cuda.Stream(device=self._sets[0][0].device)
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
-            self._eager(2)                       # warm-up outside capture
+        chunk = self._resident or self._eager
+        with torch.cuda.stream(side):            # warm-up outside capture
+            if self._resident is not None:
+                self._resident()
+            else:
+                self._eager(2)
         torch.cuda.current_stream().wait_stream(side)
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph):
-            self._eager()
+            chunk()
         for plane, value in zip(self._sets[0], saved):
             plane.copy_(value)
 

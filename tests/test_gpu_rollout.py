@@ -216,7 +216,7 @@ def test_one_launch_rollout_is_bitwise_the_eager_ticks(gpu, n, m, batch, fmt, st
     else:
         soma, dend = column_drive(batch).to(gpu), 0.1
     rollout = MatrixRollout(seeded, ticks, drive=soma, dendritic_drive=dend, trace=True)
-    assert rollout._resident is not None and rollout.graph is None
+    assert rollout._resident is not None and rollout.graph is not None
     for chunk in range(2):
         if chunk and staged:
             soma = (torch.rand(ticks, batch, n, generator=gen) * 0.4).to(gpu)
@@ -234,6 +234,31 @@ def test_one_launch_rollout_is_bitwise_the_eager_ticks(gpu, n, m, batch, fmt, st
                    dendritic_drive=dend[t].expand(batch, n) if staged else dend)
     for field in FIELDS:
         assert torch.equal(getattr(rollout, field), getattr(eager, field)), field
+
+
+@pytest.mark.parametrize("n,m", [(1024, 16_384), (2049, 30_000)])
+def test_the_captured_chunk_replays_as_run_does(gpu, n, m):
+    """``MatrixRollout.graph`` replayed by the caller is ``run()``, for the one-launch
+    chunk and for the captured ticks, over refilled inputs and eager work in between;
+    building the rollout leaves its states as seeded."""
+    print(f"case rollout graph N={n} M={m}", flush=True)
+    case = make_case(n, m, 3, gpu, kind="reference")
+    start = torch.rand(2, n, generator=torch.Generator().manual_seed(n)).to(gpu)
+    ticks = 6
+    drives = torch.rand(4, ticks, 2, n, generator=torch.Generator().manual_seed(1)).to(gpu) * 0.4
+    ran, replayed = (
+        MatrixRollout(NativeDendriticMatrixRuntime(case.topology, case.model, start.clone()),
+                      ticks, drive=drives[0].clone(), dendritic_drive=0.1, trace=True)
+        for _ in range(2))
+    assert (ran._resident is not None) == (n <= 1024) and replayed.graph is not None
+    assert torch.equal(replayed.state, start)
+    for drive in drives:
+        for rollout in (ran, replayed):
+            rollout.stage(drive)
+        ran.run()
+        replayed.graph.replay()
+        for field in (*FIELDS, "trace"):
+            assert torch.equal(getattr(ran, field), getattr(replayed, field)), field
 
 
 def test_rollouts_that_do_not_fit_use_the_graph(gpu):
