@@ -1015,7 +1015,10 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
         matrix = native and self._path == "matrix"
         # Inside a capture the scatter stays: no replay could follow the activity.
         gather = self._gather and not torch.cuda.is_current_stream_capturing()
-        out_weight = self._source_major() if not (matrix or gather) else None
+        # The product reads no copy; it is kept current for ticks captured from here.
+        out_weight = self._source_major() if not matrix else None
+        if gather:
+            out_weight = None
         topology, params = self.topology, self._parameters()
         if native:
             # One launch with pending buffers: pending[parity] holds the last tick's

@@ -501,3 +501,40 @@ def test_in_edge_product_follows_activity_weights_and_captures(gpu, always_gathe
         torch.cuda.synchronize()
     assert not native._gather
     same()
+
+
+def test_capture_after_product_ticks_streams_the_current_weights(gpu, always_gather):
+    """One eager tick on new weights is enough for a captured scatter to stream their
+    source-major copy, also while eager ticks run the in-edge product."""
+    print("case pels capture after product ticks", flush=True)
+    case = make_case(3000, 60_000, 8, gpu)
+    topology = case.topology
+    native, twin = (NativeDendriticPELSRuntime(topology, case.model,
+                                               torch.full((1, 3000), 0.1, device=gpu),
+                                               theta=0.005, policy_interval=2)
+                    for _ in range(2))
+    for tick in range(8):
+        for runtime in (native, twin):
+            runtime.step(0.3 if tick % 2 else 0.1, dendritic_drive=0.1)
+        torch.cuda.synchronize()
+    with torch.no_grad():
+        topology.in_weight.mul_(0.5)
+    for runtime in (native, twin):
+        runtime.step(0.2, dendritic_drive=0.1)
+    assert native._gather
+    read = [native.state, native.dendritic_state, native.adaptation_state, native.emitted_state]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(2):
+            native.step(0.2, dendritic_drive=0.1)
+    copy = native._prepared._out_weight[0]
+    assert copy is not None and torch.equal(
+        copy, topology.in_weight[topology.out_weight_index.long()])
+    graph.replay()
+    for _ in range(2):
+        twin.step(0.2, dendritic_drive=0.1)
+    torch.cuda.synchronize()
+    assert len(read) == 4                            # alive until the replay has read them
+    # Sums in another order: a value near theta may emit a tick earlier or later.
+    assert max_err(native.state, twin.state) <= 2e-2
+    assert float((native.state - twin.state).abs().mean()) <= 1e-5
