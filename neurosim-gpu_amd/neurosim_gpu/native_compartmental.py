@@ -746,6 +746,12 @@ class NativeDendriticMatrixRuntime(_NativeCompartments, DendriticMatrixRuntime):
 # active, and the counts cost half a microsecond per tick.
 PRODUCT_MIN_EDGES = 1_500_000
 
+# The product is left again below this share of the break-even.  At the break-even both
+# sides take the same time, at 0.8 of it the product a seventh more (N=166k, M=10M, B=1,
+# 270k active out-edges: scatter 21 us, product 23.5); without a margin activity
+# near the line would change the path, and the order of the sums, at every sample.
+PRODUCT_MARGIN = 0.8
+
 
 def product_break_even(n_edges: int, batch: int) -> float:
     """Active out-edges of a tick from which the in-edge product beats the scatter.
@@ -776,9 +782,9 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
     either way).  Reading ``persistent_current`` folds the outstanding buffer
     first, so the attribute always holds W @ emitted as in the reference;
     assigning it discards the outstanding buffer.  On a graph of at least
-    ``PRODUCT_MIN_EDGES`` edges times columns an eager tick counts its active
-    out-edges every ``policy_interval`` ticks (on the device, read back without
-    waiting), and while they exceed ``product_break_even`` the deltas propagate by
+    ``PRODUCT_MIN_EDGES`` edges times columns two eager ticks of every
+    ``policy_interval`` count their active out-edges (on the device, read back
+    without waiting), and while they exceed ``product_break_even`` the deltas propagate by
     a second launch that sums each destination's in-edges from the emitting
     sources, without atomics: the same sums in another order.  The scatter streams a
     source-major copy of the weights (M floats, rebuilt when the weights
@@ -865,7 +871,7 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
             self._activity_host = torch.zeros(slots, dtype=torch.int64, pin_memory=True)
             self._activity_counts = self._activity_host.numpy().reshape(EVENT_ACTIVITY_SLOTS,
                                                                         EVENT_ACTIVITY_STRIDE)
-            self._activity_seen = 0
+            self._activity_seen = self._counted = 0
             self._sampled = torch.cuda.Event()
         # The matrix propagation's product kernel and, for panels, its layout.
         if kernel == "panels" and (batch not in (1, 2) or not native):
@@ -908,35 +914,54 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
 
     def _policy_tick(self) -> bool:
         """Apply a finished sample and say whether this tick samples (counts its
-        active out-edges).  "auto" does so at policy ticks; the scatter of a large
-        graph (``_adaptive``) applies a sample on the first tick that finds it done."""
+        active out-edges).  "auto" does so at policy ticks.  The scatter of a large
+        graph (``_adaptive``) applies a sample on the first tick that finds it done
+        and samples two neighbouring ticks per interval, one tick later in every
+        interval, so that an input whose period divides the interval is not seen at
+        one phase only."""
         if self._activity is None:
             return False
-        phase = self._tick % self.policy_interval
+        interval, tick = self.policy_interval, self._tick
+        phase = tick % interval
         if self._adaptive:
-            due = phase == self.policy_interval // 2     # past the start state's transient
+            # The first window lies past the start state's transient.
+            first = (interval // 2 + tick // interval) % max(interval - 1, 1)
+            due = first <= phase <= first + 1
             if not due and self._sample is None:
                 return False
+            self._window_ends = phase == min(first + 1, interval - 1)
         else:
-            due = phase == 0
+            due = self._window_ends = phase == 0
             if not due:
                 return False
         if torch.cuda.is_current_stream_capturing():
             return False
         if self._sample is not None:
             if not self._sample.query():
-                return False                 # the last sample is still on its way
-            # The counters only grow: a sample is what they grew by.
+                return due and self._adaptive    # the last sample is still on its way
+            # The counters only grow: a sample is what they grew by, over its ticks.
             total = int(self._activity_counts[:, 0].sum())
-            edges, self._activity_seen = total - self._activity_seen, total
+            edges = (total - self._activity_seen) / self._sample_ticks
+            self._activity_seen = total
             if self._adaptive:
-                self._gather = edges >= product_break_even(self.topology.n_edges,
-                                                           self.state.shape[0])
+                enough = product_break_even(self.topology.n_edges, self.state.shape[0])
+                # Once on, the product stays until activity is clearly below.
+                self._gather = edges >= (PRODUCT_MARGIN * enough if self._gather else enough)
             else:
                 slots = max(self.topology.n_edges * self.state.shape[0], 1)
                 self._path = "event" if edges / slots < self.event_edge_fraction else "matrix"
             self._sample = None
         return due
+
+    def _take_sample(self) -> None:
+        """After a sampled tick: at its window's end the counters are copied to the host
+        behind it, and a later tick reads them once the copy is done."""
+        self._counted += 1
+        if self._window_ends and self._sample is None:
+            self._activity_host.copy_(self._activity, non_blocking=True)
+            self._sample_ticks, self._counted = self._counted, 0
+            self._sample = self._sampled
+            self._sample.record()
 
     def _destinations(self) -> tuple:
         """The destination-major view for the in-edge product and its bitmap."""
@@ -1062,11 +1087,7 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
                     topology.in_weight, self._current, panels)
             product()
         if sample:
-            # The counters reach the host behind this tick; a later tick reads them
-            # once the copy is done.
-            self._activity_host.copy_(self._activity, non_blocking=True)
-            self._sample = self._sampled
-            self._sample.record()
+            self._take_sample()
         if self._pending is not None:
             self._parity ^= 1
         self._tick += 1

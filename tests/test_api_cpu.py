@@ -340,3 +340,72 @@ def test_weight_storage_bytes_equal_the_published_payloads(edges, published):
         runtime = SimpleNamespace(topology=SimpleNamespace(n_edges=edges),
                                   weight_dtype=dtype, weight_format=fmt)
         assert NativeDendriticMatrixRuntime.weight_storage_bytes.fget(runtime) == published[mode]
+
+
+def follow_activity(monkeypatch, activity, ticks, interval=16, enough=1000.0, lag=0):
+    """The native PELS policy alone, its counters and event played by the host: the
+    ticks that run the in-edge product when tick t has ``activity(t)`` active edges and
+    a sample arrives ``lag`` ticks after it was taken."""
+    import numpy as np
+
+    from neurosim_gpu import native_compartmental as nc
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(nc, "product_break_even", lambda *_: enough)
+    runtime = object.__new__(nc.NativeDendriticPELSRuntime)
+    device, host = np.zeros((2, 2), np.int64), np.zeros((2, 2), np.int64)
+
+    class Host:
+        def copy_(self, source, non_blocking):
+            host[:] = source
+
+    class Event:
+        def record(self):
+            self.due = runtime._tick + lag
+
+        def query(self):
+            return runtime._tick > self.due
+
+    values = dict(_activity=device, _activity_host=Host(), _activity_counts=host, _sample=None,
+                  _activity_seen=0, _counted=0, _sampled=Event(), _adaptive=True, _gather=False,
+                  policy_interval=interval, _tick=0, state=torch.zeros(1, 4),
+                  topology=type("T", (), {"n_edges": 100, "n_neurons": 4})())
+    vars(runtime).update(values)
+    product = []
+    for tick in range(ticks):
+        sampled = runtime._policy_tick()
+        product.append(runtime._gather)
+        if sampled:
+            device[tick % 2, 0] += activity(tick)
+            runtime._take_sample()
+        runtime._tick += 1
+    return product
+
+
+@pytest.mark.parametrize("interval", [1, 2, 3, 4, 16])
+@pytest.mark.parametrize("lag", [0, 3, 40])
+def test_pels_policy_follows_steady_activity(monkeypatch, interval, lag):
+    on = follow_activity(monkeypatch, lambda t: 5000 if t < 200 else 0, 500, interval, lag=lag)
+    first = on.index(True)
+    assert first <= 2 * interval + lag + 2 and all(on[first:200])
+    # one sample of each kind may be on its way, and one window may straddle the fall
+    assert not any(on[200 + 4 * (interval + lag) + 4:])
+
+
+def test_pels_policy_sees_every_phase_of_its_input(monkeypatch):
+    """Inputs whose period divides the interval: a burst at the phase that is sampled
+    first, a pause there, and a flicker on every other tick."""
+    burst = follow_activity(monkeypatch, lambda t: 50_000 if t % 16 == 8 else 0, 4800)
+    pause = follow_activity(monkeypatch, lambda t: 0 if t % 16 == 8 else 50_000, 4800)
+    assert sum(burst) <= 0.2 * len(burst) and sum(pause) >= 0.9 * len(pause)
+    for phase in (0, 1):
+        for level, expected in ((1900, False), (2100, True)):      # means below, above 1000
+            on = follow_activity(monkeypatch, lambda t: level if t % 2 == phase else 0, 400)
+            assert set(on[40:]) == {expected}, (phase, level)
+
+
+def test_pels_policy_keeps_its_path_near_the_break_even(monkeypatch):
+    on = follow_activity(monkeypatch, lambda t: 1050 if t // 32 % 2 else 850, 1600)
+    assert sum(a != b for a, b in zip(on, on[1:])) == 1
+    below = follow_activity(monkeypatch, lambda t: 1050 if t < 200 else 750, 1600)
+    assert any(below) and not any(below[240:])
