@@ -753,21 +753,41 @@ PRODUCT_MIN_EDGES = 1_500_000
 PRODUCT_MARGIN = 0.8
 
 
-def product_break_even(n_edges: int, batch: int) -> float:
+# Most (neuron, column) pairs whose emission bitmap the product stages in LDS (batch 1
+# and 2): 64 KiB, kProductBitBytes.
+PRODUCT_BITMAP_PAIRS = 8 * 64 * 1024
+
+
+def product_break_even(topology, batch: int) -> float:
     """Active out-edges of a tick from which the in-edge product beats the scatter.
 
-    The scatter's cost is its atomics, the product's the stream of the edges, and
-    the host side of its second launch on small graphs.  Crossings measured (N, M, B,
-    thousands of active out-edges): 50k 1.5M 1, 150; 30k 2M 1, 120; 13k 1.2M 3, 110;
-    50k 4M 1, 130; 166k 10M 1, 440; 300k 15M 1, 560; 166k 25M 1, 760; 100k 4M 5, 1000;
-    and where the scatter adds runs of columns, 60k 5M 2, 190; 60k 3M 4, 350; 50k 1M 8,
-    240; 60k 3M 16, 800.  At 12-15% activity, us per eager tick, scatter / product:
-    166k 10M 1, 68 / 29; 166k 25M 1, 164 / 48; 30k 2M 1, 27 / 15; 13k 1.2M 3, 40 /
-    15; 50k 1M 8, 41 / 18."""
-    slots = n_edges * batch
-    if 2 <= batch <= 64 and batch & (batch - 1) == 0:
-        return max(200_000, 100_000 + 0.02 * slots)
-    return max(150_000, 60_000 + 0.03 * slots)
+    The scatter's cost is its atomics, about 0.05 us per thousand active out-edges
+    whatever the graph.  The product's is its edges and its rows, each form of the
+    kernel at its own rate (the bitmap in LDS; one, two or four columns per lane and
+    up to 16 columns per pass over the edges), and at least its launch, which an eager
+    tick of 14.5 us waits for.  Crossings measured / this rule, in thousands (N, M, B): bitmap
+    50k 4M 1, 125 / 126; 166k 10M 1, 333 / 345; 300k 15M 1, 489 / 555; 166k 25M 1, 652 /
+    675; 100k 5M 2, 219 / 260; 600k 10M 1, 1118 / 1120; 100k 5M 3, 633 / 560; 60k 3M 4, 338 /
+    360; 100k 4M 5, 1083 / 1090; 50k 1M 8, 250 / 263; 100k 3M 8, 686 / 641; 50k 1M 9, 622 /
+    604; 60k 3M 16, 835 / 791; 50k 1M 32, 1217 / 988.  At 12-15% activity, us per eager
+    tick, scatter / product: 166k 10M 1, 80 / 29; 166k 25M 1, 164 / 48; 30k 2M 1, 26 /
+    15; 13k 1.2M 3, 40 / 16; 50k 1M 8, 40 / 19."""
+    n, edges = topology.n_neurons, topology.n_edges
+    pairs = n * batch
+    passes = -(-batch // 16)
+    if batch <= 2 and pairs <= PRODUCT_BITMAP_PAIRS:
+        cost = 0.022 * edges + 0.75 * pairs
+    elif batch <= 4:
+        cost = 0.088 * edges + 0.40 * pairs
+    elif batch < 8:
+        cost = 0.225 * edges + 0.38 * pairs
+    elif batch == 8:
+        cost = 0.115 * edges + 0.37 * pairs
+    elif batch % 4 == 0:
+        cost = passes * (0.11 * edges + 0.48 * 16 * n)
+    else:
+        cost = passes * (0.18 * edges + 0.53 * 16 * n)
+    return max(120_000 if batch == 1 else 160_000, cost)
 
 
 class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
@@ -944,7 +964,7 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
             edges = (total - self._activity_seen) / self._sample_ticks
             self._activity_seen = total
             if self._adaptive:
-                enough = product_break_even(self.topology.n_edges, self.state.shape[0])
+                enough = product_break_even(self.topology, self.state.shape[0])
                 # Once on, the product stays until activity is clearly below.
                 self._gather = edges >= (PRODUCT_MARGIN * enough if self._gather else enough)
             else:

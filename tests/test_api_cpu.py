@@ -409,3 +409,38 @@ def test_pels_policy_keeps_its_path_near_the_break_even(monkeypatch):
     assert sum(a != b for a, b in zip(on, on[1:])) == 1
     below = follow_activity(monkeypatch, lambda t: 1050 if t < 200 else 750, 1600)
     assert any(below) and not any(below[240:])
+
+
+# Active out-edges (thousands) at which scatter and in-edge product took the same time per
+# eager tick on an MI355X: (thousands of neurons, of edges, columns, crossing).
+PELS_CROSSINGS = [
+    (20, 1500, 1, 101), (30, 2000, 1, 95), (50, 1500, 1, 146), (50, 4000, 1, 125),
+    (100, 4000, 1, 156), (100, 10000, 1, 228), (166, 4000, 1, 196), (166, 10000, 1, 333),
+    (166, 25000, 1, 652), (200, 5000, 1, 242), (300, 10000, 1, 393), (300, 15000, 1, 489),
+    (300, 20000, 1, 663), (500, 20000, 1, 1048), (530, 20000, 1, 1946), (600, 10000, 1, 1118),
+    (50, 1000, 2, 180), (60, 2500, 2, 159), (60, 5000, 2, 168), (100, 5000, 2, 219),
+    (166, 10000, 2, 568), (250, 6000, 2, 557), (300, 10000, 2, 1131), (13, 1200, 3, 130),
+    (40, 1000, 3, 188), (50, 2000, 3, 259), (100, 5000, 3, 633), (50, 500, 4, 202),
+    (50, 1000, 4, 183), (60, 3000, 4, 338), (80, 2000, 4, 318), (100, 5000, 4, 594),
+    (50, 1000, 5, 331), (100, 4000, 5, 1083), (50, 1000, 6, 341), (100, 3000, 6, 824),
+    (50, 2000, 7, 552), (30, 1000, 8, 194), (30, 1500, 8, 221), (50, 1000, 8, 250),
+    (100, 1500, 8, 507), (100, 3000, 8, 686), (30, 3000, 9, 822), (50, 1000, 9, 622),
+    (50, 1000, 11, 665), (30, 3000, 12, 526), (50, 1000, 12, 394), (20, 1000, 16, 244),
+    (40, 2000, 16, 499), (50, 500, 16, 475), (60, 3000, 16, 835), (20, 1000, 17, 617),
+    (50, 1000, 17, 1167), (20, 1000, 20, 479), (50, 1000, 20, 872), (20, 400, 24, 384),
+    (60, 3000, 24, 1830), (20, 1000, 32, 564), (50, 1000, 32, 1217), (20, 500, 33, 824),
+    (20, 400, 64, 1176)
+]
+
+
+@pytest.mark.parametrize("neurons,edges,batch,crossing", PELS_CROSSINGS)
+def test_pels_break_even_lies_near_the_measured_crossings(neurons, edges, batch, crossing):
+    """Within a third of every crossing, where the slower side costs at most about a
+    quarter more (the scatter's time grows by a twentieth of a us per thousand)."""
+    from types import SimpleNamespace
+
+    from neurosim_gpu.native_compartmental import product_break_even
+
+    topology = SimpleNamespace(n_neurons=neurons * 1000, n_edges=edges * 1000)
+    ratio = product_break_even(topology, batch) / (1000 * crossing)
+    assert 2 / 3 <= ratio <= 4 / 3, ratio
