@@ -538,3 +538,45 @@ def test_capture_after_product_ticks_streams_the_current_weights(gpu, always_gat
     # Sums in another order: a value near theta may emit a tick earlier or later.
     assert max_err(native.state, twin.state) <= 2e-2
     assert float((native.state - twin.state).abs().mean()) <= 1e-5
+
+
+@pytest.mark.parametrize("batch,pairs_over", [(1, -1), (1, 1), (2, -2), (2, 2)])
+def test_in_edge_product_at_the_bitmap_limit(gpu, always_gather, batch, pairs_over):
+    """The product just below and just above the 524288 pairs whose bitmap fits 64 KiB of
+    LDS (the bitmap form and the one that reads every edge's delta), with more lanes than
+    the bitmap form's 1024 workgroups hold, so that a group walks several rows: odd
+    numbers of neurons, empty rows, and hub rows among the last ones."""
+    from cases import model_to, standard_model
+    from neurosim_gpu import SparseTopology
+
+    n = (8 * 64 * 1024 + pairs_over) // batch
+    print(f"case pels product bitmap limit N={n} B={batch}", flush=True)
+    m = 10 * n                                       # two lanes per row: 2 N > 1024 * 512
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(n)
+    src = torch.randint(n, (m,), device=gpu, generator=gen)
+    dst = torch.randint(n - 9, (m,), device=gpu, generator=gen)
+    dst -= (dst % 7 == 3).long()                     # one row in seven is empty
+    hubs = torch.arange(4 * 3001, device=gpu)
+    src = torch.cat((src, hubs * 37 % n))
+    dst = torch.cat((dst, torch.tensor([0, n - 8, n - 2, n - 1], device=gpu)[hubs % 4]))
+    key = torch.unique(dst * n + src)
+    dst = torch.div(key, n, rounding_mode="floor")
+    src = key - dst * n
+    weight = torch.randn(key.numel(), device=gpu, generator=gen) * 0.02
+    topology = SparseTopology.from_edges(n, src, dst, weight)
+    state = torch.full((batch, n), 0.2, device=gpu)
+    native = NativeDendriticPELSRuntime(topology, model_to(standard_model(n)[0], gpu), state,
+                                        theta=0.01, policy_interval=4)
+    bursts = torch.rand((batch, n), device=gpu, generator=gen) < 0.3
+    gathered = 0
+    for tick in range(12):
+        native.step(0.2 + 0.3 * (bursts if tick % 2 else ~bursts).float(), dendritic_drive=0.1)
+        torch.cuda.synchronize()
+        gathered += native._gather
+    assert gathered >= 8
+    emitted = native.emitted_state.double()
+    assert 0.05 < float((emitted != 0.2).double().mean())
+    want = torch.zeros(batch, n, dtype=torch.float64, device=gpu)
+    want.index_add_(1, dst, emitted.index_select(1, src) * weight.double())
+    assert max_err(native.persistent_current, want.float()) <= 1e-5
