@@ -139,6 +139,10 @@ class SourceMajorWeights:
         ``version`` adds to the key (e.g. a topology weight version)."""
         if not self.enabled:
             return None
+        held = self._key
+        if (self._values is not None and weight is self._source and version == held[1]
+                and held[0][1] == (None if torch.is_inference(weight) else weight._version)):
+            return self._values
         key = (_weight_key(weight), version)
         if key != self._key or self._source is not weight:
             self._key, self._source, self._seen, self._values = key, weight, 0, None
@@ -802,9 +806,9 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
     either way).  Reading ``persistent_current`` folds the outstanding buffer
     first, so the attribute always holds W @ emitted as in the reference;
     assigning it discards the outstanding buffer.  On a graph of at least
-    ``PRODUCT_MIN_EDGES`` edges times columns two eager ticks of every
-    ``policy_interval`` count their active out-edges (on the device, read back
-    without waiting), and while they exceed ``product_break_even`` the deltas propagate by
+    ``PRODUCT_MIN_EDGES`` edges times columns one eager tick of every
+    ``policy_interval`` counts its active out-edges (on the device, read back without
+    waiting), and while they exceed ``product_break_even`` the deltas propagate by
     a second launch that sums each destination's in-edges from the emitting
     sources, without atomics: the same sums in another order.  The scatter streams a
     source-major copy of the weights (M floats, rebuilt when the weights
@@ -882,6 +886,7 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
                           and topology.n_edges * batch >= PRODUCT_MIN_EDGES)
         self._gather = False
         self._in_view = None
+        self._copied = None         # the weight version the product's ticks keep a copy of
         if self._adaptive:
             self._delta = torch.empty(batch * n, dtype=torch.float32, device=device)
         self._activity = self._activity_host = self._sample = None
@@ -891,7 +896,7 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
             self._activity_host = torch.zeros(slots, dtype=torch.int64, pin_memory=True)
             self._activity_counts = self._activity_host.numpy().reshape(EVENT_ACTIVITY_SLOTS,
                                                                         EVENT_ACTIVITY_STRIDE)
-            self._activity_seen = self._counted = 0
+            self._activity_seen, self._edges_before, self._due = 0, None, -1
             self._sampled = torch.cuda.Event()
         # The matrix propagation's product kernel and, for panels, its layout.
         if kernel == "panels" and (batch not in (1, 2) or not native):
@@ -935,63 +940,69 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
     def _policy_tick(self) -> bool:
         """Apply a finished sample and say whether this tick samples (counts its
         active out-edges).  "auto" does so at policy ticks.  The scatter of a large
-        graph (``_adaptive``) applies a sample on the first tick that finds it done
-        and samples two neighbouring ticks per interval, one tick later in every
-        interval, so that an input whose period divides the interval is not seen at
-        one phase only."""
+        graph (``_adaptive``) applies a sample on the first tick that finds it done,
+        averaged with the one before, and samples one tick per interval at a phase
+        that moves (``_next_due``), so that an input whose period divides the
+        interval is not seen at one phase only."""
         if self._activity is None:
             return False
-        interval, tick = self.policy_interval, self._tick
-        phase = tick % interval
+        tick = self._tick
         if self._adaptive:
-            # The first window lies past the start state's transient.
-            first = (interval // 2 + tick // interval) % max(interval - 1, 1)
-            due = first <= phase <= first + 1
+            if tick > self._due:
+                self._due = self._next_due(tick)
+            due = tick == self._due
             if not due and self._sample is None:
                 return False
-            self._window_ends = phase == min(first + 1, interval - 1)
         else:
-            due = self._window_ends = phase == 0
+            due = tick % self.policy_interval == 0
             if not due:
                 return False
         if torch.cuda.is_current_stream_capturing():
             return False
         if self._sample is not None:
             if not self._sample.query():
-                return due and self._adaptive    # the last sample is still on its way
-            # The counters only grow: a sample is what they grew by, over its ticks.
+                return False                 # the last sample is still on its way
+            # The counters only grow: a sample is what they grew by.
             total = int(self._activity_counts[:, 0].sum())
-            edges = (total - self._activity_seen) / self._sample_ticks
-            self._activity_seen = total
+            edges, self._activity_seen = total - self._activity_seen, total
             if self._adaptive:
+                mean = edges if self._edges_before is None else (edges + self._edges_before) / 2
+                self._edges_before = edges
                 enough = product_break_even(self.topology, self.state.shape[0])
                 # Once on, the product stays until activity is clearly below.
-                self._gather = edges >= (PRODUCT_MARGIN * enough if self._gather else enough)
+                self._gather = mean >= (PRODUCT_MARGIN * enough if self._gather else enough)
             else:
                 slots = max(self.topology.n_edges * self.state.shape[0], 1)
                 self._path = "event" if edges / slots < self.event_edge_fraction else "matrix"
             self._sample = None
         return due
 
+    def _next_due(self, tick: int) -> int:
+        """The first sampled tick from ``tick`` on: one per interval, the first past the
+        start state's transient, neighbouring ones an odd number of ticks apart (two
+        of them see both sides of a flicker)."""
+        interval = self.policy_interval
+        k = tick // interval
+        step = 1 + interval % 2
+        due = k * interval + (interval // 2 + k * step) % interval
+        if due < tick:
+            k += 1
+            due = k * interval + (interval // 2 + k * step) % interval
+        return due
+
     def _take_sample(self) -> None:
-        """After a sampled tick: at its window's end the counters are copied to the host
-        behind it, and a later tick reads them once the copy is done."""
-        self._counted += 1
-        if self._window_ends and self._sample is None:
-            self._activity_host.copy_(self._activity, non_blocking=True)
-            self._sample_ticks, self._counted = self._counted, 0
-            self._sample = self._sampled
-            self._sample.record()
+        """After a sampled tick: its counters are copied to the host behind it, and a
+        later tick reads them once the copy is done."""
+        self._activity_host.copy_(self._activity, non_blocking=True)
+        self._sample = self._sampled
+        self._sample.record()
 
     def _destinations(self) -> tuple:
         """The destination-major view for the in-edge product and its bitmap."""
-        topology = self.topology
-        view = self._in_view
-        if view is None or view[0] is not topology.in_rowptr or view[1] is not topology.in_col:
-            words = torch.empty((self._delta.numel() + 63) // 64, dtype=torch.int64,
-                                device=self._delta.device)
-            view = self._in_view = (topology.in_rowptr, topology.in_col, words)
-        return view
+        words = torch.empty((self._delta.numel() + 63) // 64, dtype=torch.int64,
+                            device=self._delta.device)
+        self._in_view = (self.topology.in_rowptr, self.topology.in_col, words)
+        return self._in_view
 
     @property
     def persistent_current(self) -> torch.Tensor:
@@ -1060,11 +1071,18 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
         matrix = native and self._path == "matrix"
         # Inside a capture the scatter stays: no replay could follow the activity.
         gather = self._gather and not torch.cuda.is_current_stream_capturing()
-        # The product reads no copy; it is kept current for ticks captured from here.
-        out_weight = self._source_major() if not matrix else None
-        if gather:
-            out_weight = None
         topology, params = self.topology, self._parameters()
+        out_weight = None
+        if gather:
+            # The product reads no copy; it is kept current for ticks captured from here
+            # (looked up only where the weights have changed: 0.2 us per tick, not 0.6).
+            kept, weight = self._copied, topology.in_weight
+            if (kept is None or weight is not kept[0] or topology.weight_version != kept[1]
+                    or (kept[2] is not None and weight._version != kept[2])):
+                self._source_major()
+                self._copied = (weight, topology.weight_version, _weight_key(weight)[1])
+        elif not matrix:
+            out_weight = self._source_major()
         if native:
             # One launch with pending buffers: pending[parity] holds the last tick's
             # scatter (or zeros) and the other is zero; the advance-only form (matrix
@@ -1072,7 +1090,10 @@ class NativeDendriticPELSRuntime(_NativeCompartments, DendriticPELSRuntime):
             tick = self._prepared
             fixed = (self.theta, topology.out_rowptr, topology.dst, topology.out_weight_index,
                      topology.in_weight)
-            in_view = self._destinations() if self._adaptive else None
+            in_view = self._in_view
+            if self._adaptive and (in_view is None or in_view[0] is not topology.in_rowptr
+                                   or in_view[1] is not topology.in_col):
+                in_view = self._destinations()
             if tick is None or not tick.matches(self.state, params, *fixed,
                                                 pending=self._pending, activity=self._activity,
                                                 in_view=in_view):

@@ -367,8 +367,9 @@ def follow_activity(monkeypatch, activity, ticks, interval=16, enough=1000.0, la
             return runtime._tick > self.due
 
     values = dict(_activity=device, _activity_host=Host(), _activity_counts=host, _sample=None,
-                  _activity_seen=0, _counted=0, _sampled=Event(), _adaptive=True, _gather=False,
-                  policy_interval=interval, _tick=0, state=torch.zeros(1, 4),
+                  _activity_seen=0, _edges_before=None, _sampled=Event(), _adaptive=True,
+                  _gather=False, policy_interval=interval, _tick=0, _due=-1,
+                  state=torch.zeros(1, 4),
                   topology=type("T", (), {"n_edges": 100, "n_neurons": 4})())
     vars(runtime).update(values)
     product = []
@@ -388,7 +389,7 @@ def test_pels_policy_follows_steady_activity(monkeypatch, interval, lag):
     on = follow_activity(monkeypatch, lambda t: 5000 if t < 200 else 0, 500, interval, lag=lag)
     first = on.index(True)
     assert first <= 2 * interval + lag + 2 and all(on[first:200])
-    # one sample of each kind may be on its way, and one window may straddle the fall
+    # a sample may be on its way, and two more are averaged with those before the fall
     assert not any(on[200 + 4 * (interval + lag) + 4:])
 
 
@@ -399,7 +400,7 @@ def test_pels_policy_sees_every_phase_of_its_input(monkeypatch):
     pause = follow_activity(monkeypatch, lambda t: 0 if t % 16 == 8 else 50_000, 4800)
     assert sum(burst) <= 0.2 * len(burst) and sum(pause) >= 0.9 * len(pause)
     for phase in (0, 1):
-        for level, expected in ((1900, False), (2100, True)):      # means below, above 1000
+        for level, expected in ((1500, False), (2100, True)):      # means 750 and 1050
             on = follow_activity(monkeypatch, lambda t: level if t % 2 == phase else 0, 400)
             assert set(on[40:]) == {expected}, (phase, level)
 
