@@ -350,9 +350,10 @@ __global__ __launch_bounds__(kThreads) void event_tick_kernel(EventArgs A) {
 // nothing for them, whatever the weight).  Lane groups as in ns_edge_rows.h, and
 // at most kProductBlocks workgroups that walk the rows.  kBits (batch 1 or 2): the
 // emitting pairs' bitmap is staged in LDS first, and an edge whose source is
-// silent costs its column index and one LDS read: a stream of 4 bytes per edge
-// with gathers for the active ones only, where the unpruned product is bound by
-// one L2 request per edge.  us per advance and product, 15% of the neurons
+// silent costs its column index and one LDS read, where the unpruned product is bound
+// by one L2 request per edge.  The weights come by the 128-byte line: with 15% of the
+// sources emitting in no order nearly every line is touched (N=166k, M=10M, B=1: 699k
+// L2 misses, 89 MB, in 23 us).  us per advance and product, 15% of the neurons
 // emitting, at 4 / 8 edges per lane in flight (the lanes per row halved to match):
 // N=166k, B=1 M=10M 29.7 / 29.0, M=25M 63.6 / 48.3; N=50k M=4M B=1 15.6 / 13.4; N=60k
 // M=3M B=16 48.8 / 44.1 (the backward's kernels lose: weight gradient at N=50k,

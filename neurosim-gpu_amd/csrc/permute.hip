@@ -7,8 +7,8 @@
 // order, one bucket being a stretch of slots that fits LDS too; then each bucket
 // is read back whole and dealt to its slots from LDS.  Both passes read and write
 // memory in runs: at 25M edges a chunk's run for a bucket is about 26 values.  The
-// two passes take 120 us there (300 MB read and written twice over, tables
-// included 500 MB: 4.2 TB/s).
+// two passes take 120 us there: 100 MB of values read and written in each, with the
+// 16-bit tables 505 MB (4.2 TB/s).
 #include <hip/hip_runtime.h>
 
 #include "neurosim_hip_layout.h"
