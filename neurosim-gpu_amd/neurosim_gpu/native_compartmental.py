@@ -142,6 +142,7 @@ class SourceMajorWeights:
         held = self._key
         if (self._values is not None and weight is self._source and version == held[1]
                 and held[0][1] == (None if torch.is_inference(weight) else weight._version)):
+            self._seen += 1
             return self._values
         key = (_weight_key(weight), version)
         if key != self._key or self._source is not weight:
