@@ -51,7 +51,7 @@ class MatrixRollout:
     ``trace=True`` also writes each tick's new somatic state into ``trace``
     ([ticks, B, N], overwritten by every replay or ``advance``): the one-launch
     rollout writes it itself, the others make one device copy per tick inside
-    the graph.  ``graph`` is the captured chunk (None with ``use_graph=False``).
+    the graph.
     """
 
     def __init__(self, runtime, ticks: int, *, drive=0.0, dendritic_drive=0.0,
@@ -91,13 +91,13 @@ class MatrixRollout:
         self.trace = (torch.empty(ticks, batch, n, dtype=torch.float32, device=state.device)
                       if trace else None)
         self.reset_from_runtime()
-        self.graph = None
+        self._graph = None
         # A network that fits a compute unit per column runs all its ticks in one
         # launch, bitwise the row-block ticks.
         self._resident = (RolloutLauncher.build(extension, self._launch, topology.in_rowptr, ticks,
                                                 self._sets[0], staged, self.trace)
                           if use_graph else None)
-        if use_graph:
+        if use_graph and self._resident is None:
             self._capture()
 
     def _eager(self, count: int | None = None) -> None:
@@ -109,21 +109,39 @@ class MatrixRollout:
                 self.trace[tick].copy_(self._sets[(tick + 1) % 2][0])
 
     def _capture(self) -> None:
-        saved = [p.clone() for p in self._sets[0]]
+        """Capture one chunk; the states, and a trace the chunk writes itself, are put
+        back after the warm-up."""
+        written = [*self._sets[0]]
+        if self._resident is not None and self.trace is not None:
+            written.append(self.trace)
+        saved = [p.clone() for p in written]
         side = torch.cuda.Stream(device=self._sets[0][0].device)
         side.wait_stream(torch.cuda.current_stream())
-        chunk = self._resident or self._eager
         with torch.cuda.stream(side):            # warm-up outside capture
             if self._resident is not None:
                 self._resident()
             else:
                 self._eager(2)
         torch.cuda.current_stream().wait_stream(side)
-        self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
-            chunk()
-        for plane, value in zip(self._sets[0], saved):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            if self._resident is not None:
+                self._resident()
+            else:
+                self._eager()
+        for plane, value in zip(written, saved):
             plane.copy_(value)
+        self._graph = graph
+
+    @property
+    def graph(self):
+        """The chunk as a HIP graph, for callers that replay it themselves (None with
+        ``use_graph=False``).  Where ``run()`` launches the chunk directly it is captured
+        on first use."""
+        if self._graph is None and self._resident is not None:
+            with torch.inference_mode():
+                self._capture()
+        return self._graph
 
     def reset_from_runtime(self) -> None:
         """Seed the rollout with the runtime's current three states."""
@@ -148,8 +166,8 @@ class MatrixRollout:
         for _ in range(repeats):
             if self._resident is not None:
                 self._resident()
-            elif self.graph is not None:
-                self.graph.replay()
+            elif self._graph is not None:
+                self._graph.replay()
             else:
                 self._eager()
 

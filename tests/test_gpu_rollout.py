@@ -259,6 +259,10 @@ def test_the_captured_chunk_replays_as_run_does(gpu, n, m):
         replayed.graph.replay()
         for field in (*FIELDS, "trace"):
             assert torch.equal(getattr(ran, field), getattr(replayed, field)), field
+    before = [getattr(ran, field).clone() for field in (*FIELDS, "trace")]
+    assert ran.graph is not None                 # may be captured only now
+    for field, value in zip((*FIELDS, "trace"), before):
+        assert torch.equal(getattr(ran, field), value), field
 
 
 def test_rollouts_that_do_not_fit_use_the_graph(gpu):
